@@ -26,6 +26,8 @@
 // Node primitives for the Roe average are recomputed from Q (the
 // primitive array holds exactly f(Q) at every node a face reads:
 // boundary rules write Q first and derive the primitives from it).
+#include <algorithm>
+
 #include "cbns_internal.hpp"
 #include "face_math.hpp"
 #include "learned.hpp"
@@ -42,10 +44,7 @@ constexpr int MARCH_Y = 4;   // lines per workgroup along the other axis
 // workgroup size of a march (the eta march: MARCH_Y wavefronts on one line)
 template <int AX>
 constexpr int march_rows() { return AX == 2 ? ZETA_ROWS : MARCH_Y; }
-#ifndef MARCH_CHUNK
-#define MARCH_CHUNK 32
-#endif
-constexpr int CHUNK = MARCH_CHUNK;  // nodes per thread along the march axis
+constexpr int CHUNK_MAX = 32;  // most nodes per thread along the march axis (march_chunk)
 #ifndef WPE_X
 #define WPE_X 3  // waves per SIMD the x-face kernel is compiled for
 #endif
@@ -163,6 +162,7 @@ struct StageArgs {
   int pmask;            // AX == 2: primitives to write (bit n: field n of rho, u, v, w, p, T)
   TroubledFaces tf;     // WENO fluxes of the march axis' troubled faces (HYB)
   TroubledFaces tf_x;   // and of the troubled xi-faces (HYB, fused xi-faces)
+  int chunk;            // nodes per thread along the march axis
 };
 
 // AX = 1: march along eta, rhs = dE + dF.  AX = 2: march along zeta, finish.
@@ -198,9 +198,9 @@ k_march(Consts c, StageArgs sa,
   if (i > upd_hi(c, 0) + (XSH ? 3 : 0) || t > upd_hi(c, ax_t)) return;
   const bool own = lane >= XL && lane < XL + march_width<AX, F>() && i <= upd_hi(c, 0);
   const int mlo = upd_lo(c, AX), mhi = upd_hi(c, AX);
-  const int m0 = mlo + blockIdx.z * CHUNK;
+  const int m0 = mlo + blockIdx.z * sa.chunk;
   if (m0 > mhi) return;
-  const int m1 = min(m0 + CHUNK, mhi + 1);
+  const int m1 = min(m0 + sa.chunk, mhi + 1);
   const long S = c.S;
   const int st = AX == 1 ? c.PX : c.PXY;
   const int base = AX == 1 ? idx(c, i, 0, t) : idx(c, i, t, 0);  // node m at base + m*st
@@ -211,22 +211,32 @@ k_march(Consts c, StageArgs sa,
   const double* __restrict__ J = met + JAC * S;
   const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
 
-  double q[6][5];  // nodes m-2 .. m+3 for the face m+1/2
+  // The face left of the chunk's first node.  Where CHUNK_MAX nodes of the
+  // line have passed (head) it is formed here, ahead of the loop; elsewhere by
+  // a first pass of the loop (m = m0 - 1) that forms the faces only.  The
+  // compiler fuses products otherwise here than in the loop, so with this rule
+  // a line's faces are those of chunks of CHUNK_MAX nodes, bit for bit,
+  // whatever the chunk: a last bit, rounded to float in the precision form or
+  // fed to the hybrid's indicator, can move a flux by a float's last bit of a
+  // shock's jump or flip a troubled flag.
+  const bool head = (m0 - mlo) % CHUNK_MAX == 0;
+  const int mb = head ? m0 : m0 - 1;  // first pass of the loop
+  double q[6][5];  // nodes m-2 .. m+3 for the face m+1/2, of the pass before
 #pragma unroll
-  for (int s = 0; s < 6; s++) load_q(Q, S, base + (m0 - 3 + s) * st, q[s]);
+  for (int s = 0; s < 6; s++) load_q(Q, S, base + (mb - 3 + s) * st, q[s]);
   // J grad xi_AX at the face's two nodes
-  int o = base + (m0 - 1) * st;
-  double ja = J[o], jb = J[o + st];
-  double ax = nX[o] * ja, ay = nY[o] * ja, az = nZ[o] * ja;
+  int o = base + (mb - 1) * st;
+  double jb = J[o + st];
+  double ax = 0.0, ay = 0.0, az = 0.0;
   double bx = nX[o + st] * jb, by = nY[o + st] * jb, bz = nZ[o + st] * jb;
-  double fprev[5];
+  double fprev[5] = {0, 0, 0, 0, 0};
   // troubled flags of faces m-1, m, m+1 (face m between nodes m and m+1)
   const uint8_t* __restrict__ fl = sa.flags;
   uint8_t t0 = 0, t1 = 0, t2 = 0;
   if (HYB) {
-    t0 = fl[base + (m0 - 2) * st];
-    t1 = fl[base + (m0 - 1) * st];
-    t2 = fl[base + m0 * st];
+    t0 = fl[base + (mb - 2) * st];
+    t1 = fl[base + (mb - 1) * st];
+    t2 = fl[base + mb * st];
   }
   // Precision form (float faces, not hybrid): the sweep carries the float
   // differences e[k] = q[k+1] - q[k] of the window's nodes and the Roe
@@ -243,13 +253,19 @@ k_march(Consts c, StageArgs sa,
       for (int n = 0; n < 5; n++) e[k][n] = (F)(q[k + 1][n] - q[k][n]);
     nl = node_t<F>(g, q_to_side(g, q[2]));
     nr = node_t<F>(g, q_to_side(g, q[3]));
-    F d[6][5];
-    dev_from_diffs(e, d);
-    face_flux_dev<F>(gt, g, d, q[2], nl, nr, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz),
-                     fprev);
-  } else {
-    stage_face<F, HYB>(g, q, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz), t0 | t1 | t2,
-                       sa.tf, base + (m0 - 1) * st, fprev);
+  }
+  if (head) {
+    const double ja = J[o];
+    ax = nX[o] * ja; ay = nY[o] * ja; az = nZ[o] * ja;
+    if constexpr (DC) {
+      F d[6][5];
+      dev_from_diffs(e, d);
+      face_flux_dev<F>(gt, g, d, q[2], nl, nr, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz),
+                       fprev);
+    } else {
+      stage_face<F, HYB>(g, q, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz), t0 | t1 | t2,
+                         sa.tf, o, fprev);
+    }
   }
   // viscous node flux of the march axis (Fv or Gv) on its offset line,
   // nodes m-1, m, m+1 of the face m+1/2 (visc_face); Ev of the xi-faces on
@@ -275,8 +291,8 @@ k_march(Consts c, StageArgs sa,
     for (int e = 0; e < 4; e++) {
       F w[4];
 #pragma unroll
-      for (int s = 0; s < 4; s++) w[s] = va[e * S + vbase + (m0 - 2 + s) * st];
-      fprev[e + 1] -= (double)visc_face(w[0], w[1], w[2], w[3]);
+      for (int s = 0; s < 4; s++) w[s] = va[e * S + vbase + (mb - 2 + s) * st];
+      if (head) fprev[e + 1] -= (double)visc_face(w[0], w[1], w[2], w[3]);
 #pragma unroll
       for (int s = 0; s < 3; s++) {
         if constexpr (VRING) vring[s][e][ty][tl] = w[s + 1];
@@ -291,11 +307,12 @@ k_march(Consts c, StageArgs sa,
   constexpr bool PF = AX == 1 && !HYB;
   double qpf[5] = {0, 0, 0, 0, 0}, jpf = 0.0, xpf = 0.0, ypf = 0.0, zpf = 0.0;
   if constexpr (PF) {
-    load_q(Q, S, base + (m0 + 3) * st, qpf);
-    const int on = base + (m0 + 1) * st;
+    load_q(Q, S, base + (mb + 3) * st, qpf);
+    const int on = base + (mb + 1) * st;
     jpf = J[on]; xpf = nX[on]; ypf = nY[on]; zpf = nZ[on];
   }
-  for (int m = m0; m < m1; m++) {
+  for (int m = mb; m < m1; m++) {
+    const bool upd = m >= m0;  // false in the first pass
     // shift the window by one node
 #pragma unroll
     for (int s = 0; s < 5; s++)
@@ -352,6 +369,12 @@ k_march(Consts c, StageArgs sa,
       bx = nX[o + st] * jb; by = nY[o + st] * jb; bz = nZ[o + st] * jb;
     }
     double f[5], fxr[5];
+    double xmx = 0.0, xmy = 0.0, xmz = 0.0;  // xi metrics of node m
+    if (XSH) {
+      xmx = met[XI_X * S + o];
+      xmy = met[XI_Y * S + o];
+      xmz = met[XI_Z * S + o];
+    }
     if (XI) {
       // the xi-face between node (i, m) and (i+1, m): stencil i-2 .. i+3
       double qx[6][5], nxx, nxy, nxz;
@@ -375,7 +398,7 @@ k_march(Consts c, StageArgs sa,
             for (int n = 0; n < 5; n++)
               qx[s][n] = s == 2 ? q[2][n] : __shfl(q[2][n], lane + s - 2);
         }
-        const double jx = xm[o] * jo, jy = xm[S + o] * jo, jz = xm[2 * S + o] * jo;
+        const double jx = xmx * jo, jy = xmy * jo, jz = xmz * jo;
         nxx = 0.5 * (jx + __shfl(jx, lane + 1));
         nxy = 0.5 * (jy + __shfl(jy, lane + 1));
         nxz = 0.5 * (jz + __shfl(jz, lane + 1));
@@ -470,6 +493,11 @@ k_march(Consts c, StageArgs sa,
         }
       }
       vr = s1;
+    }
+    if (!upd) {
+#pragma unroll
+      for (int n = 0; n < 5; n++) fprev[n] = f[n];
+      continue;
     }
     double dfx[5];  // xi-face difference (XI)
     if (XI) {
@@ -672,6 +700,44 @@ int launch_face_lists(cbns_block* b) {
   return CBNS_OK;
 }
 
+// Nodes per thread of a march over `lines` wavefront-wide lines of n nodes.
+// A thread's chunk is a serial chain of about chunk + 2 faces (its first face
+// and the window's loads come on top; one wavefront alone takes 2.1 us a node
+// in the eta march, 4.2 in the zeta march), so a block that does not fill the
+// chip (1024 SIMDs, two march wavefronts each) is cut into shorter chunks
+// until it does, and a large one into long chunks, which repeat the fewest
+// faces and window loads.  The chunk with the least
+//   (chunk + 2) x (rounds of 2048 wavefronts)
+// is taken, a round costing 1.8 (two wavefronts on a SIMD slow each other)
+// and the last one 1 if it leaves a wavefront per SIMD; since wavefronts start
+// as others end, the rounds count half as whole ones and half as a fraction.
+// From 4096 wavefronts at 32 nodes on, shorter chunks only lost.  The chunk
+// divides CHUNK_MAX (k_march, head).  Measured (FP64, eta / zeta
+// march, us, before: 32 nodes always): 24^3 58 / 110 -> 9 / 13 (1 node), 64^3
+// 58 / 152 -> 24 / 44 (4), 128x64x64 59 / 149 -> 38 / 61 (4), 128^3 viscous
+// 127 / 302 -> 138 / 247 (16), 256^3 unchanged (32).  Of 15 chunks tried on
+// each of 19 blocks the rule's is 3 % off the best on average.
+static int march_chunk(long lines, int n) {
+  constexpr long SLOTS = 2048;
+  constexpr double PAIR = 1.8;
+  auto waves = [&](int ch) { return lines * ((n + ch - 1) / ch); };
+  if (waves(CHUNK_MAX) >= 2 * SLOTS) return CHUNK_MAX;
+  int best = CHUNK_MAX;
+  double least = 1e300;
+  for (int ch = CHUNK_MAX; ch >= 1; ch /= 2) {
+    const long w = waves(ch), rest = w % SLOTS;
+    const double whole = PAIR * (double)(w / SLOTS) +
+                         (rest == 0 ? 0.0 : (rest <= SLOTS / 2 ? 1.0 : PAIR));
+    const double part = std::max(1.0, PAIR * (double)w / SLOTS) + 0.5 * PAIR;
+    const double cost = (std::min(ch, n) + 2) * 0.5 * (whole + part);
+    if (cost < least) {
+      least = cost;
+      best = ch;
+    }
+  }
+  return best;
+}
+
 template <class F, bool HYB>
 int launch_marches_eta(cbns_block* b, StageArgs& sa) {
   const Consts& c = b->c;
@@ -680,7 +746,8 @@ int launch_marches_eta(cbns_block* b, StageArgs& sa) {
   const int nm = upd_hi(c, 1) - upd_lo(c, 1) + 1;
   const int per_wave = march_width<1, F>();
   const int nwx = (ni + per_wave - 1) / per_wave;
-  dim3 grid((nwx + MARCH_Y - 1) / MARCH_Y, nt, (nm + CHUNK - 1) / CHUNK);
+  sa.chunk = march_chunk((long)nwx * nt, nm);
+  dim3 grid((nwx + MARCH_Y - 1) / MARCH_Y, nt, (nm + sa.chunk - 1) / sa.chunk);
   ProfScope ps(b, CBNS_K_MARCH_ETA);
   k_march<1, F, HYB><<<grid, dim3(MARCH_X, MARCH_Y), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
@@ -695,7 +762,9 @@ int launch_marches_zeta(cbns_block* b, StageArgs& sa) {
   const int nm = upd_hi(c, 2) - upd_lo(c, 2) + 1;
   const int per_wave = march_width<2, F>();
   constexpr int R = march_rows<2>();
-  dim3 grid((ni + per_wave - 1) / per_wave, (nt + R - 1) / R, (nm + CHUNK - 1) / CHUNK);
+  const int nwx = (ni + per_wave - 1) / per_wave;
+  sa.chunk = march_chunk((long)nwx * nt, nm);
+  dim3 grid(nwx, (nt + R - 1) / R, (nm + sa.chunk - 1) / sa.chunk);
   ProfScope ps(b, CBNS_K_MARCH_ZETA);
   k_march<2, F, HYB><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
@@ -769,7 +838,7 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
                b->rhs, c.viscous && visc_in_marches<F>() ? b->vtmp : nullptr,
                hyb ? fl + S : nullptr, hyb ? fl : nullptr, pmask,
                TroubledFaces{hyb ? b->tslot + S : nullptr, b->tflux, b->ttotal},
-               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}};
+               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, CHUNK_MAX};
   if ((rc = hyb ? launch_marches_eta<F, true>(b, sa) : launch_marches_eta<F, false>(b, sa)))
     return rc;
   if (c.viscous) {
