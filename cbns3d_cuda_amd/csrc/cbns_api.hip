@@ -129,7 +129,6 @@ int lazy_alloc(cbns_block* b, double** p, long n) {
 int ensure_stage_scratch(cbns_block* b) {
   const long S = b->c.S;
   int rc;
-  if (fused_stage_uses_face_flux() && (rc = lazy_alloc(b, &b->flux, 15 * S))) return rc;
   if (b->c.viscous && (rc = lazy_alloc(b, &b->vtmp, 12 * S))) return rc;
   if (b->c.viscous && (rc = lazy_alloc(b, &b->lam_part, visc_flux_blocks(b->c)))) return rc;
   return CBNS_OK;

@@ -366,7 +366,6 @@ long time_step_blocks(const Consts& c);
 int launch_dt_device(cbns_block* b, double cap, double* out);
 int launch_sutherland(cbns_block* b);
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout);
-bool fused_stage_uses_face_flux();
 int launch_fill(hipStream_t s, double* p, long n, double v);
 long face_count(const cbns_block* b, int axis);
 int launch_face_samples(cbns_block* b, int axis, const double* Q, float* feat, float* label);

@@ -3,25 +3,18 @@
 //   k_march<1>   lanes along i, each thread marches a chunk of nodes along
 //                eta holding the 6-node stencil and the previous face flux in
 //                registers: each node is loaded once per sweep and each face
-//                is computed once.  One of the two marches (xi_axis: the
-//                zeta march) also computes, at every node, the xi-face on its
-//                right; the left one comes from the lane below by a wavefront
-//                shuffle.  In the zeta march the xi-stencils come from the
-//                neighbouring lanes' windows and a wavefront updates 58
-//                nodes; in the eta march (the other placement) a wavefront
-//                updates 63 nodes, its lane 0 only supplies that face, and the
-//                xi-stencils are loaded (march_width).  Writes rhs = dF, or
-//                dE + dF with the xi-faces here.
-//                (FUSE_XI=0: a separate k_xfaces pass writes the xi-face
-//                fluxes to HBM and the march reads them back.)
+//                is computed once.  Writes rhs = dF.
 //   [viscous]    k_visc_fluxes (k_viscous.hip) writes the viscous node
 //                fluxes before the marches; each march subtracts their
 //                4th-order face values from its face fluxes (visc_face), so
 //                the divergence needs no pass of its own
-//   k_march<2>   the same march along zeta; adds dG, divides by J and
-//                applies the Shu-Osher stage combination, writing the stage
-//                output and its primitives (the boundary pass then only
-//                fills boundaries and ghosts).
+//   k_march<2>   the same march along zeta; at every node it also computes
+//                the xi-face on its right, from the neighbouring lanes'
+//                windows, and takes the left one from the lane below, all by
+//                wavefront shuffles.  Adds dE + dG, divides by J and applies
+//                the Shu-Osher stage combination, writing the stage output
+//                and its primitives (the boundary pass then only fills
+//                boundaries and ghosts).
 //
 // Node primitives for the Roe average are recomputed from Q (the
 // primitive array holds exactly f(Q) at every node a face reads:
@@ -37,17 +30,8 @@ namespace cbns {
 namespace {
 
 constexpr int MARCH_X = 64;  // lanes along i
-constexpr int MARCH_Y = 4;   // lines per workgroup along the other axis
-#ifndef ZETA_ROWS
-#define ZETA_ROWS 4  // the zeta march's lines along j per workgroup
-#endif
-// workgroup size of a march (the eta march: MARCH_Y wavefronts on one line)
-template <int AX>
-constexpr int march_rows() { return AX == 2 ? ZETA_ROWS : MARCH_Y; }
-constexpr int CHUNK_MAX = 32;  // most nodes per thread along the march axis (march_chunk)
-#ifndef WPE_X
-#define WPE_X 3  // waves per SIMD the x-face kernel is compiled for
-#endif
+constexpr int MARCH_Y = 4;   // wavefronts of a workgroup
+constexpr int CHUNK_MAX = 32;  // most nodes per thread along the march axis (march_cut)
 #ifndef WPE_M
 #define WPE_M 2  // waves per SIMD the march kernels are compiled for
 #endif
@@ -55,20 +39,25 @@ constexpr int CHUNK_MAX = 32;  // most nodes per thread along the march axis (ma
 #define WPE_H 2  // the same for the hybrid marches (linear faces only; three
                  // waves per SIMD measured 2-4 % slower, four spilled)
 #endif
-#ifndef FUSE_XI
-#define FUSE_XI 1  // xi-faces inside a march (no xi-face pass through HBM)
-#endif
-// The march that also forms the xi-faces: the zeta march, whose RK-update
-// traffic then overlaps the extra face work (the eta march alone is bound
-// by its face arithmetic, the zeta march by its update traffic).  Measured
-// against the eta march: +3 to +5 % of the FP64 step, +9 % of the FP32 step.
-// Both placements are supported (xi_axis 1 or 2).
-template <class F>
-constexpr int xi_axis() { return 2; }
-// nodes a march wavefront updates along i (see k_march)
-template <int AX, class F>
-constexpr int march_width() {
-  return !(FUSE_XI && AX == xi_axis<F>()) ? MARCH_X : (AX == 2 ? MARCH_X - 6 : MARCH_X - 1);
+// Halo lanes on either side of the nodes a march wavefront updates: none in
+// the eta march, 3 in the zeta march, whose xi-stencils come from the
+// neighbouring lanes.  (The zeta march has the xi-faces because its RK-update
+// traffic overlaps the extra face work; the eta march alone is bound by its
+// face arithmetic: +3 to +5 % of the FP64 step, +9 % of the FP32 step.)
+template <int AX>
+constexpr int march_halo() { return AX == 2 ? 3 : 0; }
+
+// The lines of a march (rows along i of ni updated nodes, halo nodes on either
+// side) are laid end to end and cut into wavefronts of 64 lanes; a wavefront
+// updates the lanes between its own 3 halo lanes and repeats those of its
+// neighbours.  A row's end then costs its 2 x 3 halo lanes instead of the rest
+// of a wavefront: tiles of 58 nodes on each row took 5 wavefronts for 256
+// nodes (4.5 here), 3 for 128 (2.3), 2 for 64 (1.2), and a last tile of one or
+// two nodes (176 nodes) took the zeta march from 0.60 to 0.96 ms.
+template <int AX>
+long march_wavefronts(int ni, int rows) {
+  constexpr int H = march_halo<AX>(), W = MARCH_X - 2 * H;
+  return ((long)rows * (ni + 2 * H) - 2 * H + W - 1) / W;
 }
 
 template <class T>
@@ -122,30 +111,6 @@ __device__ __forceinline__ void stage_face(const GasT<double>& g, const double q
   }
 }
 
-template <class F, bool HYB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE_X, WPE_X))) k_xfaces(Consts c, Box box, const double* __restrict__ Q,
-                                                const double* __restrict__ met,
-                                                const uint8_t* __restrict__ flags,
-                                                TroubledFaces tf,
-                                                double* __restrict__ fx) {
-  int i, j, k;
-  if (!box_node3(box, i, j, k)) return;
-  const long S = c.S;
-  const int a = idx(c, i, j, k), b = a + 1;
-  const double Ja = met[JAC * S + a], Jb = met[JAC * S + b];
-  const double nx = 0.5 * (met[XI_X * S + a] * Ja + met[XI_X * S + b] * Jb);
-  const double ny = 0.5 * (met[XI_Y * S + a] * Ja + met[XI_Y * S + b] * Jb);
-  const double nz = 0.5 * (met[XI_Z * S + a] * Ja + met[XI_Z * S + b] * Jb);
-  double q[6][5], f[5];
-#pragma unroll
-  for (int s = 0; s < 6; s++) load_q(Q, S, a + (s - 2), q[s]);
-  const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
-  const bool troubled = HYB && (flags[a - 1] | flags[a] | flags[a + 1]);
-  stage_face<F, HYB>(g, q, nx, ny, nz, troubled, tf, a, f);
-#pragma unroll
-  for (int n = 0; n < 5; n++) fx[n * S + a] = f[n];
-}
-
 struct StageArgs {
   double dt;
   const double* dtp;    // dt on the device (the folded time step) or null: use dt
@@ -154,53 +119,46 @@ struct StageArgs {
   const double* Qn;     // level-n state (stages 2, 3)
   const double* Qin;    // stage input (stencil source)
   double* Qout;         // stage output
-  const double* fx;     // xi-face fluxes (AX == 1)
-  double* rhs;          // dE + dF (+ viscous)
+  double* rhs;          // dF
   const void* vf;       // viscous node fluxes Ev, Fv, Gv (12 fields of the face type) or null
   const uint8_t* flags; // troubled faces of the march axis (HYB)
-  const uint8_t* flags_x;  // troubled xi-faces (HYB, fused xi-faces)
+  const uint8_t* flags_x;  // troubled xi-faces (HYB, AX == 2)
   int pmask;            // AX == 2: primitives to write (bit n: field n of rho, u, v, w, p, T)
   TroubledFaces tf;     // WENO fluxes of the march axis' troubled faces (HYB)
-  TroubledFaces tf_x;   // and of the troubled xi-faces (HYB, fused xi-faces)
-  int chunk;            // nodes per thread along the march axis
+  TroubledFaces tf_x;   // and of the troubled xi-faces (HYB, AX == 2)
+  int parts;            // chunks per CHUNK_MAX nodes of a line
 };
 
-// AX = 1: march along eta, rhs = dE + dF.  AX = 2: march along zeta, finish.
+// AX = 1: march along eta, rhs = dF.  AX = 2: march along zeta with the
+// xi-faces, finish.
 template <int AX, class F, bool HYB>
-__global__ void __launch_bounds__(MARCH_X * march_rows<AX>())
+__global__ void __launch_bounds__(MARCH_X * MARCH_Y)
 __attribute__((amdgpu_waves_per_eu(HYB ? WPE_H : WPE_M, HYB ? WPE_H : WPE_M)))
-k_march(Consts c, StageArgs sa,
-                                                            const double* __restrict__ met) {
-  constexpr bool XI = AX == xi_axis<F>() && FUSE_XI;
+k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
+  constexpr bool XI = AX == 2;
   // the update's time step; a NaN step (non-physical state) leaves the
   // stage output unwritten, and the caller reports it
   const double dt = AX == 2 && sa.dtp ? *sa.dtp : sa.dt;
   if (AX == 2 && !(dt == dt)) return;
   const int ax_t = AX == 1 ? 2 : 1;  // transverse axis other than i
   const int lane = threadIdx.x;
-  // XI in the eta march: a wavefront updates 63 nodes, its lane 0 sits one
-  // node to the left and loads its xi-stencils.  XI in the zeta march (XSH):
-  // the xi-stencils come from the neighbouring lanes' march windows by
-  // wavefront shuffles, so a wavefront holds 3 nodes on either side of the
-  // 58 it updates (the zeta march is bound by its memory instructions, the
-  // eta march by arithmetic).
-  constexpr bool XSH = XI && AX == 2;
-  constexpr int XL = XSH ? 3 : (XI ? 1 : 0);  // lanes left of the first updated node
-  // eta march: the workgroup's wavefronts take adjacent tiles of one line
-  // along i, so each step along eta reads whole rows of the fields (-9 % for
-  // the FP64 eta march, -12 % FP32).  zeta march: wavefronts on adjacent
-  // lines (its 58-node tiles would leave idle wavefronts on a line)
-  constexpr bool ROWS = AX == 1;
-  const int i = upd_lo(c, 0) - XL +
-                (ROWS ? blockIdx.x * MARCH_Y + threadIdx.y : blockIdx.x) * march_width<AX, F>() +
-                lane;
-  const int t = upd_lo(c, ax_t) + (ROWS ? blockIdx.y : blockIdx.y * march_rows<AX>() + threadIdx.y);
-  if (i > upd_hi(c, 0) + (XSH ? 3 : 0) || t > upd_hi(c, ax_t)) return;
-  const bool own = lane >= XL && lane < XL + march_width<AX, F>() && i <= upd_hi(c, 0);
+  // the workgroup's wavefronts follow each other along the lines, so each
+  // step of the march reads whole rows of the fields (against wavefronts on
+  // adjacent lines -9 % for the FP64 eta march, -12 % FP32)
+  constexpr int H = march_halo<AX>(), W = MARCH_X - 2 * H;
+  const int ni = upd_hi(c, 0) - upd_lo(c, 0) + 1;
+  const unsigned slot = (blockIdx.x * blockDim.y + threadIdx.y) * W + lane;
+  const unsigned row = slot / (unsigned)(ni + 2 * H);
+  const int at = (int)(slot - row * (unsigned)(ni + 2 * H)) - H;  // node of the row's updated ones
+  const int i = upd_lo(c, 0) + at;
+  const int t = upd_lo(c, ax_t) + (int)row;
+  if (t > upd_hi(c, ax_t)) return;
+  const bool own = lane >= H && lane < H + W && at >= 0 && at < ni;
   const int mlo = upd_lo(c, AX), mhi = upd_hi(c, AX);
-  const int m0 = mlo + blockIdx.z * sa.chunk;
+  const int mseg = mlo + CHUNK_MAX * (int)blockIdx.z, part = blockIdx.y;
+  const int m0 = mseg + CHUNK_MAX * part / sa.parts;
   if (m0 > mhi) return;
-  const int m1 = min(m0 + sa.chunk, mhi + 1);
+  const int m1 = min(mseg + CHUNK_MAX * (part + 1) / sa.parts, mhi + 1);
   const long S = c.S;
   const int st = AX == 1 ? c.PX : c.PXY;
   const int base = AX == 1 ? idx(c, i, 0, t) : idx(c, i, t, 0);  // node m at base + m*st
@@ -219,7 +177,7 @@ k_march(Consts c, StageArgs sa,
   // whatever the chunk: a last bit, rounded to float in the precision form or
   // fed to the hybrid's indicator, can move a flux by a float's last bit of a
   // shock's jump or flip a troubled flag.
-  const bool head = (m0 - mlo) % CHUNK_MAX == 0;
+  const bool head = part == 0;
   const int mb = head ? m0 : m0 - 1;  // first pass of the loop
   double q[6][5];  // nodes m-2 .. m+3 for the face m+1/2, of the pass before
 #pragma unroll
@@ -275,13 +233,13 @@ k_march(Consts c, StageArgs sa,
   const F* __restrict__ ve = static_cast<const F*>(sa.vf);
   const F* __restrict__ va = VIS ? ve + (long)(4 * AX) * S : nullptr;
   const int vbase = AX == 1 ? idx(c, i + vsh, 0, t + vsh) : idx(c, i + vsh, t + vsh, 0);
-  const int ebase = idx(c, i, t + vsh, vsh);  // XSH: Ev of node m at ebase + m*st
+  const int ebase = idx(c, i, t + vsh, vsh);  // Ev of node m at ebase + m*st (XI)
   // The window (nodes m-1, m, m+1) is held in registers, or, in the FP64
   // zeta march, whose registers the xi-faces take, in a per-thread LDS ring
   // (slot vr holds node m-1, the next two slots the others; no thread reads
   // another's entries, so no barrier).
-  constexpr bool VRING = AX == 2 && XSH && sizeof(F) == sizeof(double) && !HYB;
-  constexpr int RR = VRING ? march_rows<AX>() : 1;
+  constexpr bool VRING = AX == 2 && sizeof(F) == sizeof(double) && !HYB;
+  constexpr int RR = VRING ? MARCH_Y : 1;
   __shared__ F vring[VRING ? 3 : 1][4][RR][VRING ? MARCH_X : 1];
   const int ty = VRING ? threadIdx.y : 0, tl = VRING ? lane : 0;
   F vw[3][4];
@@ -326,12 +284,12 @@ k_march(Consts c, StageArgs sa,
     } else {
       load_q(Q, S, o + 3 * st, q[5]);
     }
-    F vn[4], ev[4];  // viscous flux of node m+2 along the axis; Ev of node m (XSH)
+    F vn[4], ev[4];  // viscous flux of node m+2 along the axis; Ev of node m (XI)
     if (VIS) {
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         vn[e] = va[e * S + vbase + (m + 2) * st];
-        if constexpr (XSH) ev[e] = ve[e * S + ebase + m * st];
+        if constexpr (XI) ev[e] = ve[e * S + ebase + m * st];
       }
     }
     if constexpr (DC) {
@@ -349,7 +307,7 @@ k_march(Consts c, StageArgs sa,
     // their latency overlaps it; with FP64 faces and the xi-faces in this
     // march they are fetched where they are used (hoisted they would push
     // the kernel past 256 VGPRs)
-    constexpr bool HOIST = AX == 2 && !(XI && sizeof(F) == sizeof(double)) && !HYB;
+    constexpr bool HOIST = AX == 2 && sizeof(F) != sizeof(double) && !HYB;
     double rin[5], qnv[5];
     if (HOIST) {
 #pragma unroll
@@ -370,59 +328,36 @@ k_march(Consts c, StageArgs sa,
     }
     double f[5], fxr[5];
     double xmx = 0.0, xmy = 0.0, xmz = 0.0;  // xi metrics of node m
-    if (XSH) {
+    if (XI) {
       xmx = met[XI_X * S + o];
       xmy = met[XI_Y * S + o];
       xmz = met[XI_Z * S + o];
     }
-    if (XI) {
+    if constexpr (XI) {
       // the xi-face between node (i, m) and (i+1, m): stencil i-2 .. i+3
-      double qx[6][5], nxx, nxy, nxz;
-      bool tx = false;
-      const double* __restrict__ xm = met + XI_X * S;
-      if constexpr (XSH) {
-        // every lane takes part in the shuffles
-        if constexpr (HYB) {
-          // linear xi-face from the neighbouring lanes' values, one
-          // component at a time (six values live, not the whole stencil)
+      // (every lane takes part in the shuffles)
+      double qx[6][5];
+      if constexpr (HYB) {
+        // linear xi-face from the neighbouring lanes' values, one
+        // component at a time (six values live, not the whole stencil)
 #pragma unroll
-          for (int n = 0; n < 5; n++) {
-            const double v = q[2][n];
-            linear_lr<F>(__shfl(v, lane - 2), __shfl(v, lane - 1), v, __shfl(v, lane + 1),
-                         __shfl(v, lane + 2), __shfl(v, lane + 3), qx[0][n], qx[1][n]);
-          }
-        } else if constexpr (!DC) {
-#pragma unroll
-          for (int s = 0; s < 6; s++)
-#pragma unroll
-            for (int n = 0; n < 5; n++)
-              qx[s][n] = s == 2 ? q[2][n] : __shfl(q[2][n], lane + s - 2);
+        for (int n = 0; n < 5; n++) {
+          const double v = q[2][n];
+          linear_lr<F>(__shfl(v, lane - 2), __shfl(v, lane - 1), v, __shfl(v, lane + 1),
+                       __shfl(v, lane + 2), __shfl(v, lane + 3), qx[0][n], qx[1][n]);
         }
-        const double jx = xmx * jo, jy = xmy * jo, jz = xmz * jo;
-        nxx = 0.5 * (jx + __shfl(jx, lane + 1));
-        nxy = 0.5 * (jy + __shfl(jy, lane + 1));
-        nxz = 0.5 * (jz + __shfl(jz, lane + 1));
-        if (HYB) {
-          const int fo = sa.flags_x[o];
-          tx = (__shfl(fo, lane - 1) | fo | __shfl(fo, lane + 1)) != 0;
-        }
-      } else {
+      } else if constexpr (!DC) {
 #pragma unroll
-        for (int s = 0; s < 6; s++) {
-          if (s == 2) {
+        for (int s = 0; s < 6; s++)
 #pragma unroll
-            for (int n = 0; n < 5; n++) qx[2][n] = q[2][n];
-          } else {
-            load_q(Q, S, o + (s - 2), qx[s]);
-          }
-        }
-        const double Ja = jo, Jb = J[o + 1];
-        nxx = 0.5 * (xm[o] * Ja + xm[o + 1] * Jb);
-        nxy = 0.5 * (xm[S + o] * Ja + xm[S + o + 1] * Jb);
-        nxz = 0.5 * (xm[2 * S + o] * Ja + xm[2 * S + o + 1] * Jb);
-        tx = HYB && (sa.flags_x[o - 1] | sa.flags_x[o] | sa.flags_x[o + 1]);
+          for (int n = 0; n < 5; n++)
+            qx[s][n] = s == 2 ? q[2][n] : __shfl(q[2][n], lane + s - 2);
       }
-      if constexpr (XSH && DC) {
+      const double jx = xmx * jo, jy = xmy * jo, jz = xmz * jo;
+      const double nxx = 0.5 * (jx + __shfl(jx, lane + 1));
+      const double nxy = 0.5 * (jy + __shfl(jy, lane + 1));
+      const double nxz = 0.5 * (jz + __shfl(jz, lane + 1));
+      if constexpr (DC) {
         // the float difference to lane+1's node, the differences of lanes
         // -2..+2 and lane+1's Roe inputs, by shuffles
         F ex[5], ec[5][5];
@@ -441,7 +376,9 @@ k_march(Consts c, StageArgs sa,
         F dx[6][5];
         dev_from_diffs(ec, dx);
         face_flux_dev<F>(gt, g, dx, q[2], nl, xr, nxx, nxy, nxz, fxr);
-      } else if constexpr (XSH && HYB) {
+      } else if constexpr (HYB) {
+        const int fo = sa.flags_x[o];
+        const bool tx = (__shfl(fo, lane - 1) | fo | __shfl(fo, lane + 1)) != 0;
         // qx[0], qx[1]: the reconstructed left and right states
         lf_flux(g, q_to_side(g, qx[1]), q_to_side(g, qx[0]), nxx, nxy, nxz, fxr);
         if (tx) {
@@ -450,16 +387,14 @@ k_march(Consts c, StageArgs sa,
           for (int n = 0; n < 5; n++) fxr[n] = sa.tf_x.flux[n * sa.tf_x.stride + sl];
         }
       } else {
-        stage_face<F, HYB>(g, qx, nxx, nxy, nxz, tx, sa.tf_x, o, fxr);
+        stage_face<F, HYB>(g, qx, nxx, nxy, nxz, false, sa.tf_x, o, fxr);
       }
-      if constexpr (XSH) {
-        if (VIS) {
+      if (VIS) {
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const F v = ev[e];
-            fxr[e + 1] -= (double)visc_face(__shfl(v, lane - 1), v, __shfl(v, lane + 1),
-                                            __shfl(v, lane + 2));
-          }
+        for (int e = 0; e < 4; e++) {
+          const F v = ev[e];
+          fxr[e + 1] -= (double)visc_face(__shfl(v, lane - 1), v, __shfl(v, lane + 1),
+                                          __shfl(v, lane + 2));
         }
       }
     }
@@ -504,19 +439,9 @@ k_march(Consts c, StageArgs sa,
 #pragma unroll
       for (int n = 0; n < 5; n++) dfx[n] = fxr[n] - __shfl_up(fxr[n], 1);
     }
-    if (AX == 1 && XI) {
-#pragma unroll
-      for (int n = 0; n < 5; n++)
-        if (own) sa.rhs[n * S + o] = dfx[n] + (f[n] - fprev[n]);
-    } else if (AX == 1 && FUSE_XI) {  // xi-faces in the zeta march
+    if (AX == 1) {
 #pragma unroll
       for (int n = 0; n < 5; n++) sa.rhs[n * S + o] = f[n] - fprev[n];
-    } else if (AX == 1) {
-#pragma unroll
-      for (int n = 0; n < 5; n++) {
-        const double* fxn = sa.fx + n * S;
-        sa.rhs[n * S + o] = (fxn[o] - fxn[o - 1]) + (f[n] - fprev[n]);
-      }
     } else {
       if (!HOIST) {
 #pragma unroll
@@ -700,73 +625,65 @@ int launch_face_lists(cbns_block* b) {
   return CBNS_OK;
 }
 
-// Nodes per thread of a march over `lines` wavefront-wide lines of n nodes.
-// A thread's chunk is a serial chain of about chunk + 2 faces (its first face
-// and the window's loads come on top; one wavefront alone takes 2.1 us a node
-// in the eta march, 4.2 in the zeta march), so a block that does not fill the
-// chip (1024 SIMDs, two march wavefronts each) is cut into shorter chunks
-// until it does, and a large one into long chunks, which repeat the fewest
-// faces and window loads.  The chunk with the least
-//   (chunk + 2) x (rounds of 2048 wavefronts)
-// is taken, a round costing 1.8 (two wavefronts on a SIMD slow each other)
-// and the last one 1 if it leaves a wavefront per SIMD; since wavefronts start
-// as others end, the rounds count half as whole ones and half as a fraction.
-// From 4096 wavefronts at 32 nodes on, shorter chunks only lost.  The chunk
-// divides CHUNK_MAX (k_march, head).  Measured (FP64, eta / zeta
-// march, us, before: 32 nodes always): 24^3 58 / 110 -> 9 / 13 (1 node), 64^3
-// 58 / 152 -> 24 / 44 (4), 128x64x64 59 / 149 -> 38 / 61 (4), 128^3 viscous
-// 127 / 302 -> 138 / 247 (16), 256^3 unchanged (32).  Of 15 chunks tried on
-// each of 19 blocks the rule's is 3 % off the best on average.
-static int march_chunk(long lines, int n) {
+// How a march over `lines` wavefronts and n nodes along its axis is cut: the
+// chunks per CHUNK_MAX nodes.  A thread's chunk is a serial chain of about
+// chunk + 1 faces (its first face and the window's loads come on top; one
+// wavefront alone takes 2.1 us a node in the eta march, 4.2 in the zeta march),
+// so a block that does not fill the chip (1024 SIMDs, two march wavefronts
+// each) is cut into shorter chunks until it does, and a large one into long
+// chunks, which repeat the fewest faces and window loads.  The cut with the
+// least
+//   (chunk + 1) x (rounds of 2048 wavefronts)
+// is taken, a round costing 1.8 (two wavefronts on a SIMD slow each other) and
+// the last one 1 if it leaves a wavefront per SIMD; since wavefronts start as
+// others end, the rounds count half as whole ones and half as a fraction.  Of
+// 15 cuts tried on each of 45 blocks (24^3 to 224^3, three forms) the rule's is
+// 1.6 % off the best on average, 14 % at worst.  Measured (FP64, eta / zeta
+// march, us, before: 32 nodes always): 24^3 58 / 110 -> 9 / 14, 64^3 58 / 152
+// -> 18 / 38, 128x64x64 59 / 149 -> 28 / 63, 128^3 viscous 127 / 302 -> 101 /
+// 215; 256^3 keeps 32.
+struct MarchCut {
+  int parts;   // chunks per CHUNK_MAX nodes
+  long waves;  // wavefronts in all
+};
+static MarchCut march_cut(long lines, int n) {
   constexpr long SLOTS = 2048;
   constexpr double PAIR = 1.8;
-  auto waves = [&](int ch) { return lines * ((n + ch - 1) / ch); };
-  if (waves(CHUNK_MAX) >= 2 * SLOTS) return CHUNK_MAX;
-  int best = CHUNK_MAX;
+  MarchCut best{1, 0};
   double least = 1e300;
-  for (int ch = CHUNK_MAX; ch >= 1; ch /= 2) {
-    const long w = waves(ch), rest = w % SLOTS;
+  for (int p = 1; p <= CHUNK_MAX; p++) {
+    const int len = std::min((CHUNK_MAX + p - 1) / p, n);
+    long chunks = (long)(n / CHUNK_MAX) * p;
+    for (int s = 0; s < p && CHUNK_MAX * s / p < n % CHUNK_MAX; s++) chunks++;
+    const long w = lines * chunks, rest = w % SLOTS;
     const double whole = PAIR * (double)(w / SLOTS) +
                          (rest == 0 ? 0.0 : (rest <= SLOTS / 2 ? 1.0 : PAIR));
-    const double part = std::max(1.0, PAIR * (double)w / SLOTS) + 0.5 * PAIR;
-    const double cost = (std::min(ch, n) + 2) * 0.5 * (whole + part);
+    const double cost = (len + 1) * (whole + std::max(1.0, PAIR * (double)w / SLOTS));
     if (cost < least) {
       least = cost;
-      best = ch;
+      best = {p, w};
     }
   }
   return best;
 }
 
-template <class F, bool HYB>
-int launch_marches_eta(cbns_block* b, StageArgs& sa) {
+template <int AX, class F, bool HYB>
+int launch_march(cbns_block* b, StageArgs& sa) {
   const Consts& c = b->c;
+  const int ax_t = AX == 1 ? 2 : 1;
   const int ni = upd_hi(c, 0) - upd_lo(c, 0) + 1;
-  const int nt = upd_hi(c, 2) - upd_lo(c, 2) + 1;
-  const int nm = upd_hi(c, 1) - upd_lo(c, 1) + 1;
-  const int per_wave = march_width<1, F>();
-  const int nwx = (ni + per_wave - 1) / per_wave;
-  sa.chunk = march_chunk((long)nwx * nt, nm);
-  dim3 grid((nwx + MARCH_Y - 1) / MARCH_Y, nt, (nm + sa.chunk - 1) / sa.chunk);
-  ProfScope ps(b, CBNS_K_MARCH_ETA);
-  k_march<1, F, HYB><<<grid, dim3(MARCH_X, MARCH_Y), 0, b->stream>>>(c, sa, b->met);
-  CBNS_HIP(b, hipGetLastError());
-  return CBNS_OK;
-}
-
-template <class F, bool HYB>
-int launch_marches_zeta(cbns_block* b, StageArgs& sa) {
-  const Consts& c = b->c;
-  const int ni = upd_hi(c, 0) - upd_lo(c, 0) + 1;
-  const int nt = upd_hi(c, 1) - upd_lo(c, 1) + 1;
-  const int nm = upd_hi(c, 2) - upd_lo(c, 2) + 1;
-  const int per_wave = march_width<2, F>();
-  constexpr int R = march_rows<2>();
-  const int nwx = (ni + per_wave - 1) / per_wave;
-  sa.chunk = march_chunk((long)nwx * nt, nm);
-  dim3 grid(nwx, (nt + R - 1) / R, (nm + sa.chunk - 1) / sa.chunk);
-  ProfScope ps(b, CBNS_K_MARCH_ZETA);
-  k_march<2, F, HYB><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
+  const int nt = upd_hi(c, ax_t) - upd_lo(c, ax_t) + 1;
+  const int nm = upd_hi(c, AX) - upd_lo(c, AX) + 1;
+  const long nw = march_wavefronts<AX>(ni, nt);
+  const MarchCut cut = march_cut(nw, nm);
+  sa.parts = cut.parts;
+  // up to a wavefront per SIMD: workgroups of one, over all CUs (24^3 zeta
+  // march 17.3 -> 15.8 us); above, neighbours along the lines share a CU's L1
+  // (128^3 zeta march 215 us, 252 with single wavefronts)
+  const int R = cut.waves <= 1024 ? 1 : MARCH_Y;
+  const dim3 grid((unsigned)((nw + R - 1) / R), sa.parts, (nm + CHUNK_MAX - 1) / CHUNK_MAX);
+  ProfScope ps(b, AX == 1 ? CBNS_K_MARCH_ETA : CBNS_K_MARCH_ZETA);
+  k_march<AX, F, HYB><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
 }
@@ -777,13 +694,7 @@ int viscous_part(cbns_block* b, double* lam, int parts) {
                                      : launch_viscous_f32(b, b->vtmp, b->rhs, lam, parts);
 }
 
-// The marches take the viscous divergence in face form (visc_face) when the
-// zeta march holds the xi-faces; otherwise k_visc_div subtracts it from the
-// right-hand side between the marches.
 constexpr int TFULL_EVERY = 8;  // steps between indicator passes while a list overflows
-
-template <class F>
-constexpr bool visc_in_marches() { return FUSE_XI && xi_axis<F>() == 2; }
 
 // One fused stage: [indicator and face lists (hybrid, when due)], viscous
 // flux pass, eta march, zeta march.  The flux pass reads only the stage
@@ -793,7 +704,6 @@ template <class F>
 int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout,
                 bool hyb_form) {
   const Consts& c = b->c;
-  double* fx = b->flux;  // first 5 face arrays
   int rc = CBNS_OK;
   if (hyb_form) {
     // once per step on the stage-1 input (or every ind_every steps, or at
@@ -817,46 +727,25 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
   if (hyb && (rc = launch_weno_lists<F>(b, qin))) return rc;
   const long S = c.S;
   const uint8_t* fl = hyb ? b->flags : nullptr;
-  if (!FUSE_XI) {
-    Box box;
-    for (int a = 0; a < 3; a++) {
-      box.lo[a] = upd_lo(c, a);
-      box.n[a] = upd_hi(c, a) - upd_lo(c, a) + 1;
-    }
-    box.lo[0] = periodic(c, 0) ? -1 : 0;
-    box.n[0] = c.IM - 1 + (periodic(c, 0) ? 2 : 0);  // faces -1..N-1 or 0..N-2
-    ProfScope ps(b, CBNS_K_XFACES);
-    const TroubledFaces tx{b->tslot, b->tflux, b->ttotal};
-    if (hyb)
-      k_xfaces<F, true><<<box_grid(box), box_block(), 0, b->stream>>>(c, box, qin, b->met, fl, tx, fx);
-    else
-      k_xfaces<F, false><<<box_grid(box), box_block(), 0, b->stream>>>(c, box, qin, b->met, fl, tx, fx);
-    CBNS_HIP(b, hipGetLastError());
-  }
   const int pmask = stage_prim_mask(b, stage);
-  StageArgs sa{dt, b->dt_fold ? b->red + 2 : nullptr, stage, b->prim, b->Q, qin, qout, fx,
-               b->rhs, c.viscous && visc_in_marches<F>() ? b->vtmp : nullptr,
+  StageArgs sa{dt, b->dt_fold ? b->red + 2 : nullptr, stage, b->prim, b->Q, qin, qout,
+               b->rhs, c.viscous ? b->vtmp : nullptr,
                hyb ? fl + S : nullptr, hyb ? fl : nullptr, pmask,
                TroubledFaces{hyb ? b->tslot + S : nullptr, b->tflux, b->ttotal},
-               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, CHUNK_MAX};
-  if ((rc = hyb ? launch_marches_eta<F, true>(b, sa) : launch_marches_eta<F, false>(b, sa)))
+               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1};
+  if ((rc = hyb ? launch_march<1, F, true>(b, sa) : launch_march<1, F, false>(b, sa)))
     return rc;
-  if (c.viscous) {
-    if (!visc_in_marches<F>() && (rc = viscous_part<F>(b, nullptr, 2))) return rc;
-    if (lam) {
-      ProfScope ps(b, CBNS_K_DT);
-      if ((rc = launch_dt_from_partials(b, lam, (int)visc_flux_blocks(c), b->dt_cap, b->red + 2)))
-        return rc;
-    }
+  if (lam) {
+    ProfScope ps(b, CBNS_K_DT);
+    if ((rc = launch_dt_from_partials(b, lam, (int)visc_flux_blocks(c), b->dt_cap, b->red + 2)))
+      return rc;
   }
   if (hyb) {
     sa.flags = fl + 2 * S;
     sa.tf.slot = b->tslot + 2 * S;
   }
-  return hyb ? launch_marches_zeta<F, true>(b, sa) : launch_marches_zeta<F, false>(b, sa);
+  return hyb ? launch_march<2, F, true>(b, sa) : launch_march<2, F, false>(b, sa);
 }
-
-bool fused_stage_uses_face_flux() { return !FUSE_XI; }
 
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout) {
   const bool hyb = (b->form & CBNS_FORM_HYBRID) != 0;

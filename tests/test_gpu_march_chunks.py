@@ -1,10 +1,11 @@
 """The marches cut a line into chunks whose length depends on the block's size
-(march_chunk, csrc/k_fused.hip).  Every face is formed from the same values by
+(march_cut, csrc/k_fused.hip).  Every face is formed from the same values by
 the same operations whatever the chunk, given its position along the line
 modulo 32, so a periodic block that repeats a
 small one of 32 nodes a line along eta and zeta takes the small block's step
-bit for bit: the small block runs chunks of 1 or 2 nodes, the larger ones 4 to
-32, with and without a shorter last chunk.
+bit for bit: the small block runs chunks of 1 node, the larger ones up to 32.
+The rows along xi are laid end to end over the wavefronts, so row ends fall on
+every lane.
 """
 import numpy as np
 import pytest
@@ -43,9 +44,8 @@ def start(case, form, met=None, q=None):
 
 @pytest.mark.parametrize("viscous", [0, 1])
 @pytest.mark.parametrize("form", [FORM_FP64, FORM_FP32, FORM_FP32 | FORM_HYBRID])
-@pytest.mark.parametrize("reps", [2, 3, 5, 8])
-def test_repeated_block_steps_alike(reps, form, viscous):
-    im = 67  # two tiles along xi, the second ragged
+@pytest.mark.parametrize("im,reps", [(67, 2), (67, 3), (67, 5), (67, 8), (5, 3), (58, 2), (129, 2)])
+def test_repeated_block_steps_alike(im, reps, form, viscous):
     small = start(cases.smooth_box(im, N0, N0, viscous=viscous), form)
     try:
         met, q = small.get_field(F_MET, 10), small.get_field(F_Q, 5)
