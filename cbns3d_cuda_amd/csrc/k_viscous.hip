@@ -25,12 +25,20 @@
 // lanes by wavefront shuffles (LDS crossbar) instead of 16 loads per node,
 // and the eta-derivatives from a plane buffer in LDS that holds the
 // workgroup's rows and two rows on either side.
-// With its stencils loaded, the flux pass waited on the vector-memory
-// pipeline (address and data units ~90 % busy at 256^3) rather than on HBM
-// bytes; the shuffles and the plane buffer cut its loads per node from 46 to
-// 18.  The divergence pass keeps its loads: there the shuffles cost 30
-// VGPRs, two of its six waves per SIMD and 20 % of its time, and a plane
-// buffer for Fv saved nothing (it is bound by its HBM bytes).
+// The flux pass streams 14 fields and writes 12: 0.78 ms at 256^3 for those
+// alone (a probe of the same streams in the same order, 4.4 TB/s), 1.02 ms for
+// the pass, FP32 0.82; what is left is the re-read of the halo rows and planes.
+// Its loads are issued together, ahead of the plane's barrier and its
+// shuffles: with a branch around each load and each one-sided stencil the
+// compiler waited for them one by one, and for the previous plane's stores
+// (us, before and now: 32^3 26 -> 11, 64^3 34 -> 25, 193x61x33 with reference
+// axes 60 -> 37, 128^3 135 -> 134, 256^3 1036 -> 1023; FP32 131x75x53 50 -> 38,
+// 128^3 119 -> 117, 256^3 815 -> 817).  Loading the metrics a plane ahead too
+// took 182 VGPRs and was 5 % slower at 128^3; the workgroups of an XCD on
+// neighbouring tiles (its L2 then holds their halos) made no difference.
+// The divergence pass keeps its loads: there the shuffles cost 30 VGPRs, two of
+// its six waves per SIMD and 20 % of its time, and a plane buffer for Fv saved
+// nothing (it is bound by its HBM bytes).
 #include "cbns_internal.hpp"
 
 namespace cbns {
@@ -47,33 +55,54 @@ constexpr int VROWS = VISC_ROWS;
 #ifndef VISC_FLUX_ROWS
 #define VISC_FLUX_ROWS 4  // flux-pass workgroup rows along j
 #endif
-#ifndef VISC_FLUX_CHUNK
-#define VISC_FLUX_CHUNK 8  // flux-pass nodes along k per thread
-#endif
+// Flux-pass nodes along k per thread.  A chunk is a chain of about one memory
+// latency a plane (2 us on an idle chip, 4 planes of lead-in on top), so the
+// best length is short: 5 of 1, 2, 3, 4, 5, 6, 8, 12, 16, 32 at 64^3 to 256^3
+// (128^3 FP64 134 us, 137 at 4, 143 at 12; 256^3 1023, 1040 at 8, 1064 at 12),
+// 2 where 5 would leave fewer than 448 workgroups (32^3: 11 us, 16 at 5).
+constexpr int VISC_FLUX_CHUNK = 5, VISC_FLUX_CHUNK_SMALL = 2;
 constexpr int FROWS = VISC_FLUX_ROWS;
 
-// 4th-order derivative along axis a at node m of the viscous range:
-// one-sided at the two outermost layers of a reference axis
-// (src/gradient_kernel.cu:162-253), central with wrapped ghosts otherwise.
-__device__ __forceinline__ double dgrad(const Consts& c, int a, int m, const double* __restrict__ f,
-                                        int st) {
-  if (!periodic(c, a)) {
-    const int p = m + 2, ne = axis_n(c, a) + 4;
+// The sums below name their fused operations, so their last bits do not depend
+// on how the compiler arranges the code around them (in the precision form a
+// float's last bit shows in the step's result).
+
+// 4th-order central difference from the values at -2, -1, +1, +2
+__device__ __forceinline__ double central4(double a, double b, double d, double e) {
+  return fma(-1.0 / 12.0, e, fma(2.0 / 3.0, d, fma(1.0 / 12.0, a, -(2.0 / 3.0 * b))));
+}
+
+// a0 b0 + a1 b1 + a2 b2
+template <class T>
+__device__ __forceinline__ T dot3(T a0, T b0, T a1, T b1, T a2, T b2) {
+  return fma(a2, b2, fma(a0, b0, a1 * b1));
+}
+
+// 4th-order derivatives of the four fields f at node offset o on one of the two
+// outermost layers of a reference axis (one-sided, src/gradient_kernel.cu:
+// 162-253): position p of the ne nodes of the viscous range along the axis, p
+// = 0, 1, ne - 2 or ne - 1, st between neighbours.  All 20 values are loaded
+// before any is used: one latency, not one per field.
+__device__ __forceinline__ void dedge(const double* const f[4], int o, int p, int ne, int st,
+                                      double d[4]) {
+  const int first = p == 0 ? 0 : (p == 1 ? -1 : (p == ne - 2 ? -3 : -4));
+  double v[4][5];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int s = 0; s < 5; s++) v[q][s] = f[q][o + (first + s) * st];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const double* w = v[q];
     if (0 == p)
-      return -25.0 / 12.0 * f[0] + 4.0 * f[st] - 3.0 * f[2 * st] + (4.0 / 3.0) * f[3 * st] -
-             0.25 * f[4 * st];
-    if (1 == p)
-      return -5.0 / 6.0 * f[0] - 0.25 * f[-st] + 1.5 * f[st] - 0.5 * f[2 * st] +
-             (1.0 / 12.0) * f[3 * st];
-    if (ne - 2 == p)
-      return (5.0 / 6.0) * f[0] - 1.0 / 12.0 * f[-3 * st] + 0.5 * f[-2 * st] - 1.5 * f[-st] +
-             0.25 * f[st];
-    if (ne - 1 == p)
-      return (25.0 / 12.0) * f[0] + 0.25 * f[-4 * st] - 4.0 / 3.0 * f[-3 * st] +
-             3.0 * f[-2 * st] - 4.0 * f[-st];
+      d[q] = -25.0 / 12.0 * w[0] + 4.0 * w[1] - 3.0 * w[2] + (4.0 / 3.0) * w[3] - 0.25 * w[4];
+    else if (1 == p)
+      d[q] = -5.0 / 6.0 * w[1] - 0.25 * w[0] + 1.5 * w[2] - 0.5 * w[3] + (1.0 / 12.0) * w[4];
+    else if (ne - 2 == p)
+      d[q] = (5.0 / 6.0) * w[3] - 1.0 / 12.0 * w[0] + 0.5 * w[1] - 1.5 * w[2] + 0.25 * w[4];
+    else
+      d[q] = (25.0 / 12.0) * w[4] + 0.25 * w[0] - 4.0 / 3.0 * w[1] + 3.0 * w[2] - 4.0 * w[3];
   }
-  return (1.0 / 12.0) * f[-2 * st] - 2.0 / 3.0 * f[-st] + (2.0 / 3.0) * f[st] -
-         1.0 / 12.0 * f[2 * st];
 }
 
 // xi-neighbours of a lane's value: n = v at i-2, i-1, i+1, i+2 (meaningful
@@ -87,26 +116,16 @@ __device__ __forceinline__ void xi_neighbours(V v, V n[4]) {
   n[3] = __shfl(v, lane + 2);
 }
 
-// d/dxi of v at node i from the neighbouring lanes (every lane takes part);
-// the one-sided layers of a reference axis read memory (dgrad, from f at the
-// node) where `node` says the lane's row is in the array
-__device__ __forceinline__ double dxi(const Consts& c, int i, double v,
-                                      const double* __restrict__ f, bool node) {
+// d/dxi of v at the node from the neighbouring lanes (every lane takes part)
+__device__ __forceinline__ double dxi(double v) {
   double nb[4];
   xi_neighbours(v, nb);
-  const double d =
-      (1.0 / 12.0) * nb[0] - 2.0 / 3.0 * nb[1] + (2.0 / 3.0) * nb[2] - 1.0 / 12.0 * nb[3];
-  // (only the four outer nodes -2, -1, IM, IM+1 of the viscous range: the
-  // halo lanes beyond them hold no node of the range)
-  if (node && !periodic(c, 0) && (i == -2 || i == -1 || i == c.IM || i == c.IM + 1))
-    return dgrad(c, 0, i, f, 1);
-  return d;
+  return central4(nb[0], nb[1], nb[2], nb[3]);
 }
 
-// 4th-order central difference from a 5-plane window (same arithmetic as
-// dgrad's central branch)
+// 4th-order central difference from a 5-plane window
 __device__ __forceinline__ double dwin(const double w[5]) {
-  return (1.0 / 12.0) * w[0] - 2.0 / 3.0 * w[1] + (2.0 / 3.0) * w[3] - 1.0 / 12.0 * w[4];
+  return central4(w[0], w[1], w[3], w[4]);
 }
 
 // The node's three viscous flux vectors E[d] = J grad xi_d . [tau; u.tau - q]
@@ -128,7 +147,7 @@ __device__ __forceinline__ double visc_node_fluxes(const Consts& c, const double
   for (int a = 0; a < 4; a++) {
     const T d0 = (T)du[a][0], d1 = (T)du[a][1], d2 = (T)du[a][2];
 #pragma unroll
-    for (int b = 0; b < 3; b++) g[a][b] = d0 * (T)m[b] + d1 * (T)m[3 + b] + d2 * (T)m[6 + b];
+    for (int b = 0; b < 3; b++) g[a][b] = dot3(d0, (T)m[b], d1, (T)m[3 + b], d2, (T)m[6 + b]);
   }
   const double mu_d = (1.0 + c.C_T_inf) / (T_l + c.C_T_inf) * sqrt(T_l * T_l * T_l);
   const T mr = (T)(mu_d * c.Re_inv);
@@ -136,7 +155,7 @@ __device__ __forceinline__ double visc_node_fluxes(const Consts& c, const double
   T tau[3][3];
 #pragma unroll
   for (int a = 0; a < 3; a++) {
-    tau[a][a] = mr * (T(2) * g[a][a] - third2);
+    tau[a][a] = mr * fma(T(2), g[a][a], -third2);
 #pragma unroll
     for (int b = a + 1; b < 3; b++) tau[a][b] = tau[b][a] = mr * (g[a][b] + g[b][a]);
   }
@@ -144,49 +163,16 @@ __device__ __forceinline__ double visc_node_fluxes(const Consts& c, const double
   T e[3];  // u . tau - q
 #pragma unroll
   for (int b = 0; b < 3; b++)
-    e[b] = (T)uvw[0] * tau[0][b] + (T)uvw[1] * tau[1][b] + (T)uvw[2] * tau[2][b] - mq * g[3][b];
+    e[b] = fma(-mq, g[3][b], dot3((T)uvw[0], tau[0][b], (T)uvw[1], tau[1][b], (T)uvw[2], tau[2][b]));
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const T nx = (T)(m[3 * d + 0] * m[JAC]), ny = (T)(m[3 * d + 1] * m[JAC]);
     const T nz = (T)(m[3 * d + 2] * m[JAC]);
 #pragma unroll
-    for (int a = 0; a < 3; a++) E[d][a] = nx * tau[0][a] + ny * tau[1][a] + nz * tau[2][a];
-    E[d][3] = nx * e[0] + ny * e[1] + nz * e[2];
+    for (int a = 0; a < 3; a++) E[d][a] = dot3(nx, tau[0][a], ny, tau[1][a], nz, tau[2][a]);
+    E[d][3] = dot3(nx, e[0], ny, e[1], nz, e[2]);
   }
   return mu_d;
-}
-
-// Fluxes of node (i, j, k) stored to vf (Ev, Fv, Gv: 4 fields each).
-// win[f][s]: field f (u,v,w,T) at k-2+s; dx[f], de[f]: d/dxi, d/deta of
-// field f; m: the node's metrics.
-template <class T>
-__device__ __forceinline__ void visc_fluxes_node(const Consts& c, int i, int j, int k,
-                                                 const double win[4][5],
-                                                 const double dx[4], const double de[4],
-                                                 const double m[10],
-                                                 const double* __restrict__ prim,
-                                                 T* __restrict__ vf) {
-  const long S = c.S;
-  const int o = idx(c, i, j, k);
-  const int sz = c.PXY;
-  // zeta: the register window, except at the one-sided outer layers of a
-  // reference axis
-  const bool zc = periodic(c, 2) || (k >= 0 && k <= c.KM - 1);
-  const int pf[4] = {P_U, P_V, P_W, P_T};
-  double du[4][3];
-#pragma unroll
-  for (int f = 0; f < 4; f++) {
-    du[f][0] = dx[f];
-    du[f][1] = de[f];
-    du[f][2] = zc ? dwin(win[f]) : dgrad(c, 2, k, prim + pf[f] * S + o, sz);
-  }
-  const double uvw[3] = {win[0][2], win[1][2], win[2][2]};
-  T E[3][4];
-  visc_node_fluxes<T>(c, du, uvw, win[3][2], m, E);
-#pragma unroll
-  for (int d = 0; d < 3; d++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) vf[(long)(4 * d + e) * S + o] = E[d][e];
 }
 
 // The workgroup's rows (64 x FROWS lanes, one row of j per wavefront) and
@@ -203,7 +189,7 @@ static_assert(FROWS >= 4, "the halo rows are loaded by the first four wavefronts
 // stencils read and take part in the barriers).  false for the whole
 // workgroup past the tile count.
 __device__ inline bool visc_flux_lane(const TileMarch& t, int& i, int& j, int& k0, int& k1,
-                                      bool& has, bool& own, bool& row_in) {
+                                      bool& own) {
   const unsigned nb = (unsigned)t.ntx * t.nty * t.nkc;
   const unsigned per = (nb + N_XCD - 1) / N_XCD;
   const unsigned lb = (blockIdx.x % N_XCD) * per + blockIdx.x / N_XCD;
@@ -212,9 +198,7 @@ __device__ inline bool visc_flux_lane(const TileMarch& t, int& i, int& j, int& k
   const unsigned ty = r % t.nty, kc = r / t.nty;
   const int lane = (int)threadIdx.x;
   const int ti = (int)tx * (BOX_X - 2 * t.xh) - t.xh + lane, tj = ty * t.rows + threadIdx.y;
-  row_in = tj < t.box.n[1];
-  has = ti < t.box.n[0] + t.xh;
-  own = row_in && lane >= t.xh && lane < BOX_X - t.xh && ti < t.box.n[0];
+  own = tj < t.box.n[1] && lane >= t.xh && lane < BOX_X - t.xh && ti < t.box.n[0];
   i = t.box.lo[0] + ti;
   j = t.box.lo[1] + tj;
   k0 = t.box.lo[2] + (int)kc * t.chunk;
@@ -225,7 +209,9 @@ __device__ inline bool visc_flux_lane(const TileMarch& t, int& i, int& j, int& k
 // LAM: also the spectral-radius maximum of the workgroup's nodes in
 // [0, IM) x [0, JM) x [0, KM) (node_lambda, the time step's per-node term),
 // written to lam_part[workgroup]; NaN if any node's is NaN.
-template <class T, bool LAM>
+// REF: the block has a reference axis (one-sided derivatives at its two outer
+// layers); a periodic block's kernel holds no branch on the position.
+template <class T, bool LAM, bool REF>
 __global__ void __launch_bounds__(64 * FROWS) k_visc_fluxes(Consts c, TileMarch tm,
                                                      const double* __restrict__ prim,
                                                      const double* __restrict__ met,
@@ -233,73 +219,101 @@ __global__ void __launch_bounds__(64 * FROWS) k_visc_fluxes(Consts c, TileMarch 
                                                      double* __restrict__ lam_part) {
   __shared__ double plane[2][4][VPLANE_ROWS][BOX_X];
   int i = 0, j = 0, k0 = 0, k1 = 0;
-  bool has = false, own = false, row_in = false;
-  if (!visc_flux_lane(tm, i, j, k0, k1, has, own, row_in)) return;
+  bool own = false;
+  if (!visc_flux_lane(tm, i, j, k0, k1, own)) return;
   const int lane = threadIdx.x, ty = threadIdx.y;
-  // the lane's row is loaded if it lies in the array (j >= -2 > -G always)
-  const bool has_row = has && j < c.JM + G;
   // halo row of this wavefront (the first four): j0-2, j0-1, j0+FROWS, j0+FROWS+1
   const int hr = ty < 2 ? ty : ty + FROWS;
   const int jh = j - ty - 2 + hr;
-  const bool halo = ty < 4, has_halo = halo && has && jh < c.JM + G;
-  // eta-stencil from the plane buffer, except at the one-sided outer layers
-  // of a reference axis
-  const bool ec = periodic(c, 1) || (j >= 0 && j <= c.JM - 1);
+  const bool halo = FROWS == 4 || ty < 4;
   double lam = -INFINITY;
   int nan_seen = 0;
   const bool lam_line = LAM && own && i >= 0 && i < c.IM && j >= 0 && j < c.JM;
   const long S = c.S;
   const int sz = c.PXY;
   const double* f0[4] = {prim + P_U * S, prim + P_V * S, prim + P_W * S, prim + P_T * S};
-  const int base = idx(c, i, j, 0), hbase = idx(c, i, jh, 0);
-  double win[4][5];
+  // lanes and rows past the array load its last ones (their values feed no
+  // node of the box)
+  const int ic = min(i, c.IM + G - 1);
+  const int base = idx(c, ic, min(j, c.JM + G - 1), 0);
+  const int hbase = idx(c, ic, min(jh, c.JM + G - 1), 0);
+  double win[4][5], hn[4];
 #pragma unroll
-  for (int f = 0; f < 4; f++)
+  for (int f = 0; f < 4; f++) {
 #pragma unroll
-    for (int s = 0; s < 4; s++) win[f][s + 1] = has_row ? f0[f][base + (k0 - 2 + s) * sz] : 0.0;
-  // the halo rows are fetched one plane ahead (plane k1 <= KM + 2 lies in
-  // the array), so the barrier does not wait on a load of its own iteration
-  // (the metrics too cost a wavefront per SIMD and ran slower)
-  double hn[4];
-#pragma unroll
-  for (int f = 0; f < 4; f++) hn[f] = has_halo ? f0[f][hbase + k0 * sz] : 0.0;
+    for (int s = 0; s < 4; s++) win[f][s + 1] = f0[f][base + (k0 - 2 + s) * sz];
+    hn[f] = f0[f][hbase + k0 * sz];
+  }
   for (int k = k0; k < k1; k++) {
-    double dx[4], de[4], hv[4];
-    const int pb = k & 1;
-#pragma unroll
-    for (int f = 0; f < 4; f++) {
-      hv[f] = hn[f];
-      hn[f] = has_halo ? f0[f][hbase + (k + 1) * sz] : 0.0;
-    }
+    // every load of the plane up front (the halo rows of the next plane, which
+    // the barrier would wait for)
+    double hv[4], m[10], rp[2] = {1.0, 1.0};
 #pragma unroll
     for (int f = 0; f < 4; f++) {
 #pragma unroll
       for (int s = 0; s < 4; s++) win[f][s] = win[f][s + 1];
-      win[f][4] = has_row ? f0[f][base + (k + 2) * sz] : 0.0;
-      dx[f] = dxi(c, i, win[f][2], f0[f] + base + k * sz, has_row);
+      win[f][4] = f0[f][base + (k + 2) * sz];
+      hv[f] = hn[f];
+      hn[f] = f0[f][hbase + (k + 1) * sz];
+    }
+#pragma unroll
+    for (int q = 0; q < 10; q++) m[q] = met[q * S + base + k * sz];
+    if (LAM) {
+      rp[0] = prim[P_RHO * S + base + k * sz];
+      rp[1] = prim[P_P * S + base + k * sz];
+    }
+    const int o = base + k * sz;
+    const int pb = k & 1;
+    double du[4][3];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
       plane[pb][f][ty + 2][lane] = win[f][2];
       if (halo) plane[pb][f][hr][lane] = hv[f];
     }
+#pragma unroll
+    for (int f = 0; f < 4; f++) du[f][0] = dxi(win[f][2]);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
+    // keeps the metric loads ahead of the barrier (they would sink to their use)
 #pragma unroll
-    for (int f = 0; f < 4; f++)
-      de[f] = ec ? (1.0 / 12.0) * plane[pb][f][ty][lane] - 2.0 / 3.0 * plane[pb][f][ty + 1][lane] +
-                       (2.0 / 3.0) * plane[pb][f][ty + 3][lane] -
-                       1.0 / 12.0 * plane[pb][f][ty + 4][lane]
-                 : (own ? dgrad(c, 1, j, f0[f] + base + k * sz, c.PX) : 0.0);
-    if (own) {
-      double m[10];
+    for (int q = 0; q < 10; q++) asm volatile("" : "+v"(m[q]));
 #pragma unroll
-      for (int q = 0; q < 10; q++) m[q] = met[q * S + base + k * sz];
-      visc_fluxes_node<T>(c, i, j, k, win, dx, de, m, prim, vf);
-      if (LAM && lam_line && k >= 0 && k < c.KM) {
-        // u, v, w, T and the metrics from the registers, rho and p loaded
-        const int o = base + k * sz;
-        const double sl = node_lambda_v(c, prim[P_RHO * S + o], win[0][2], win[1][2], win[2][2],
-                                        prim[P_P * S + o], win[3][2], m);
-        if (isnan(sl)) nan_seen = 1;
-        else lam = fmax(lam, sl);
+    for (int f = 0; f < 4; f++) {
+      du[f][1] = central4(plane[pb][f][ty][lane], plane[pb][f][ty + 1][lane],
+                          plane[pb][f][ty + 3][lane], plane[pb][f][ty + 4][lane]);
+      du[f][2] = dwin(win[f]);
+    }
+    if (REF && own) {
+      double d[4];
+      if (!periodic(c, 0) && (i < 0 || i >= c.IM)) {
+        dedge(f0, o, i + 2, c.IM + 4, 1, d);
+#pragma unroll
+        for (int f = 0; f < 4; f++) du[f][0] = d[f];
       }
+      if (!periodic(c, 1) && (j < 0 || j >= c.JM)) {
+        dedge(f0, o, j + 2, c.JM + 4, c.PX, d);
+#pragma unroll
+        for (int f = 0; f < 4; f++) du[f][1] = d[f];
+      }
+      if (!periodic(c, 2) && (k < 0 || k >= c.KM)) {
+        dedge(f0, o, k + 2, c.KM + 4, sz, d);
+#pragma unroll
+        for (int f = 0; f < 4; f++) du[f][2] = d[f];
+      }
+    }
+    const double uvw[3] = {win[0][2], win[1][2], win[2][2]};
+    T E[3][4];
+    visc_node_fluxes<T>(c, du, uvw, win[3][2], m, E);
+    if (LAM && lam_line && k >= 0 && k < c.KM) {
+      const double sl = node_lambda_v(c, rp[0], uvw[0], uvw[1], uvw[2], rp[1], win[3][2], m);
+      if (isnan(sl)) nan_seen = 1;
+      else lam = fmax(lam, sl);
+    }
+    if (own) {
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) vf[(long)(4 * d + e) * S + o] = E[d][e];
     }
   }
   if (LAM) {
@@ -373,7 +387,9 @@ static TileMarch visc_flux_tiles(const Consts& c) {
     vb.lo[a] = -2;
     vb.n[a] = axis_n(c, a) + 4;
   }
-  return tile_march(vb, VISC_FLUX_CHUNK, FROWS, 2);
+  const TileMarch tm = tile_march(vb, VISC_FLUX_CHUNK, FROWS, 2);
+  if ((long)tm.ntx * tm.nty * tm.nkc >= 448) return tm;
+  return tile_march(vb, VISC_FLUX_CHUNK_SMALL, FROWS, 2);
 }
 
 long visc_flux_blocks(const Consts& c) { return (long)tile_march_blocks(visc_flux_tiles(c)); }
@@ -389,12 +405,10 @@ int viscous(cbns_block* b, T* vf, double* out, int mode, double* lam_part, int p
     ProfScope ps(b, CBNS_K_VISC_FLUX);
     const TileMarch tm = visc_flux_tiles(c);
     const dim3 grid(tile_march_blocks(tm)), block(BOX_X, FROWS);
-    if (lam_part)
-      k_visc_fluxes<T, true><<<grid, block, 0, b->stream>>>(c, tm, b->prim, b->met, vf,
-                                                            lam_part);
-    else
-      k_visc_fluxes<T, false><<<grid, block, 0, b->stream>>>(c, tm, b->prim, b->met, vf,
-                                                             nullptr);
+    const bool ref = !periodic(c, 0) || !periodic(c, 1) || !periodic(c, 2);
+    const auto kern = lam_part ? (ref ? k_visc_fluxes<T, true, true> : k_visc_fluxes<T, true, false>)
+                               : (ref ? k_visc_fluxes<T, false, true> : k_visc_fluxes<T, false, false>);
+    kern<<<grid, block, 0, b->stream>>>(c, tm, b->prim, b->met, vf, lam_part);
     CBNS_HIP(b, hipGetLastError());
   }
   if (!(parts & 2)) return CBNS_OK;
