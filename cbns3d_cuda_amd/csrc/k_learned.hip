@@ -10,8 +10,11 @@
 //   k_mlp_forward       logits of a feature batch
 //   k_mlp_grad          weighted logistic loss and its gradient: forward and
 //                       backward on the matrix cores; weight gradients are
-//                       16x16x16 products over faces after an LDS transpose
-//   k_mlp_adam          Adam update of the fp32 parameters
+//                       16x16x16 products over faces after an LDS transpose;
+//                       one row of sums per workgroup
+//   k_mlp_sum           the rows' sums: gradient and loss
+//   k_mlp_adam          Adam update of the fp32 parameters and their bf16
+//                       operand tiles
 //   k_mlp_pack          fp32 parameters -> bf16 operand tiles
 #include <cmath>
 #include <cstring>
@@ -144,18 +147,36 @@ __device__ __forceinline__ float softplus(float s) {
   return s > 0.0f ? s + log1pf(expf(-s)) : log1pf(expf(s));
 }
 
-// One wavefront takes 64 samples per iteration (four 16-face tiles).
-// grad (MLP_NPARAM floats) and loss_sum are accumulated atomically.
-__global__ void __launch_bounds__(256) k_mlp_grad(MlpDev w, const float* __restrict__ X,
-                                                  const float* __restrict__ Y, long n,
-                                                  float w_pos, float inv_n, int iters,
-                                                  float* __restrict__ grad,
-                                                  float* __restrict__ loss_sum) {
-  __shared__ short tr[4][4 * 32 * 16];  // per wave: dz2, h1, dz1, x as [row][16 faces]
-  __shared__ float gacc[MLP_NPARAM + 1];
+// sum over the 16 lanes of a row of lanes, in every lane (rotations within it)
+__device__ __forceinline__ float row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
+  return v;
+}
+
+// A wavefront takes a tile of 16 samples per iteration.  Each workgroup writes
+// its sums to its own row of `part`; k_mlp_sum adds the rows, so no sum depends
+// on the order the workgroups end in.  A sample's chain (load, four dependent
+// matrix products, exp, LDS transpose, four more) is latency, so the 4,096 tiles
+// of a 65,536-sample batch go to 2,048 wavefronts, the two a SIMD holds at 192
+// VGPRs (held to 128 for four it spilled: 111 us).  12 us at 65,536 samples and
+// 4 for the rows' sum; 41 before, with float atomics in LDS and 256 atomics on
+// each of the 2,146 sums, after a fill.
+constexpr int GRAD_WAVES = 8;          // of a workgroup
+constexpr int GRAD_BLOCKS = 256;       // most workgroups
+constexpr int GRAD_ROW = 2176;         // floats of a row: gradient, loss, padding
+static_assert(MLP_NPARAM + 1 <= GRAD_ROW, "a row holds the gradient and the loss");
+
+__global__ void __launch_bounds__(64 * GRAD_WAVES) k_mlp_grad(
+    MlpDev w, const float* __restrict__ X, const float* __restrict__ Y, long n, float w_pos,
+    float inv_n, int iters, float* __restrict__ part) {
+  // per wavefront: dz2, h1, dz1, x as [row][16 faces] in the loop, its sums
+  // (parameter order, then the loss) after it
+  __shared__ float acc[GRAD_WAVES][GRAD_ROW];
+  static_assert(GRAD_ROW * sizeof(float) >= 4 * 32 * 16 * sizeof(short), "the tiles fit");
   const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, lq = l >> 4, lr = l & 15;
-  for (int t = threadIdx.x; t <= MLP_NPARAM; t += blockDim.x) gacc[t] = 0.0f;
-  __syncthreads();
   bf16x4 a1[4], a2[4], a2t[4];
 #pragma unroll
   for (int t = 0; t < 4; t++) {
@@ -179,11 +200,11 @@ __global__ void __launch_bounds__(256) k_mlp_grad(MlpDev w, const float* __restr
   f32x4 gW1[2][2] = {{zero, zero}, {zero, zero}}, gW2[2][2] = {{zero, zero}, {zero, zero}};
   float gb1[2][4] = {}, gb2[2][4] = {}, gw3[2][4] = {};
   float gb3 = 0.0f, lsum = 0.0f;
-  short* T = tr[wv];
+  short* T = reinterpret_cast<short*>(acc[wv]);
   for (int it = 0; it < iters; it++) {
-    const long chunk = ((long)blockIdx.x * 4 + wv) + (long)it * gridDim.x * 4;
-    for (int ft = 0; ft < 4; ft++) {
-      const long smp = chunk * 64 + 16 * ft + lr;
+    {
+      const long tile = (long)blockIdx.x * GRAD_WAVES + wv + (long)it * gridDim.x * GRAD_WAVES;
+      const long smp = tile * 16 + lr;
       const bool valid = smp < n;
       bf16x4 x[2];
       if (valid) {
@@ -275,7 +296,9 @@ __global__ void __launch_bounds__(256) k_mlp_grad(MlpDev w, const float* __restr
       wave_sync_lds();
     }
   }
-  // block reduction in LDS, then one global atomic per parameter
+  // every wavefront's sums, then the workgroup's row: plain stores and one sum
+  // per parameter (float atomics in LDS on these 58 values a lane took 30 us)
+  float* A = acc[wv];
 #pragma unroll
   for (int r = 0; r < 2; r++)
 #pragma unroll
@@ -283,47 +306,73 @@ __global__ void __launch_bounds__(256) k_mlp_grad(MlpDev w, const float* __restr
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int row = 16 * r + 4 * lq + v, col = 16 * cc + lr;
-        atomicAdd(&gacc[MLP_W2 + row * MLP_HID + col], gW2[r][cc][v]);
-        atomicAdd(&gacc[MLP_W1 + row * MLP_IN + col], gW1[r][cc][v]);
+        A[MLP_W2 + row * MLP_HID + col] = gW2[r][cc][v];
+        A[MLP_W1 + row * MLP_IN + col] = gW1[r][cc][v];
       }
 #pragma unroll
   for (int t = 0; t < 2; t++)
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const int row = 16 * t + 4 * lq + v;
-      atomicAdd(&gacc[MLP_B1 + row], gb1[t][v]);
-      atomicAdd(&gacc[MLP_B2 + row], gb2[t][v]);
-      atomicAdd(&gacc[MLP_W3 + row], gw3[t][v]);
+      const float s1 = row_sum(gb1[t][v]), s2 = row_sum(gb2[t][v]), s3 = row_sum(gw3[t][v]);
+      if (lr == 0) {
+        A[MLP_B1 + row] = s1;
+        A[MLP_B2 + row] = s2;
+        A[MLP_W3 + row] = s3;
+      }
     }
-  if (lq == 0) {
-    atomicAdd(&gacc[MLP_B3], gb3);
-    atomicAdd(&gacc[MLP_NPARAM], lsum);
+  gb3 = row_sum(gb3);  // lanes 0..15 hold the samples' terms
+  lsum = row_sum(lsum);
+  if (l == 0) {
+    A[MLP_B3] = gb3;
+    A[MLP_NPARAM] = lsum;
   }
   __syncthreads();
-  for (int t = threadIdx.x; t < MLP_NPARAM; t += blockDim.x) atomicAdd(&grad[t], gacc[t]);
-  if (threadIdx.x == 0) atomicAdd(loss_sum, gacc[MLP_NPARAM]);
+  for (int t = threadIdx.x; t <= MLP_NPARAM; t += blockDim.x) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < GRAD_WAVES; w++) sum += acc[w][t];
+    part[(long)blockIdx.x * GRAD_ROW + t] = sum;
+  }
 }
 
-// Adam on the fp32 parameters; W1's two padding input columns stay zero.
-__global__ void k_mlp_adam(float* __restrict__ P, const float* __restrict__ grad,
-                           float* __restrict__ m, float* __restrict__ v, float lr, float b1,
-                           float b2, float eps, float c1, float c2) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= MLP_NPARAM) return;
-  if (t < MLP_B1 && (t % MLP_IN) >= MLP_NFEAT) return;
-  const float g = grad[t];
-  const float mt = b1 * m[t] + (1.0f - b1) * g;
-  const float vt = b2 * v[t] + (1.0f - b2) * g * g;
-  m[t] = mt;
-  v[t] = vt;
-  P[t] -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
+// out[t] = sum of part[row][t] over the rows, t <= MLP_NPARAM: 64 sums per
+// workgroup, 16 wavefronts on every 16th row, eight loads in flight.  host (or
+// null): the same in host memory, so that no copy follows.
+constexpr int SUM_WAVES = 16;
+__global__ void __launch_bounds__(64 * SUM_WAVES) k_mlp_sum(const float* __restrict__ part,
+                                                            int rows, float* __restrict__ out,
+                                                            float* __restrict__ host) {
+  __shared__ float acc[SUM_WAVES][64];
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, t = (int)blockIdx.x * 64 + l;
+  float a = 0.0f;
+  constexpr int U = 8;
+  for (int r0 = wv; r0 < rows; r0 += U * SUM_WAVES) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int r = r0 + u * SUM_WAVES;
+      v[u] = r < rows ? part[(long)r * GRAD_ROW + t] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) a += v[u];
+  }
+  acc[wv][l] = a;
+  __syncthreads();
+  if (wv == 0 && t <= MLP_NPARAM) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < SUM_WAVES; r++) sum += acc[r][l];
+    out[t] = sum;
+    if (host) host[t] = sum;
+  }
 }
 
 // A-operand tiles t = 2 * row_tile + k_tile: lane l item e holds
-// M[16 row_tile + l % 16][16 k_tile + 4 (l / 16) + e].
-__global__ void k_mlp_pack(const float* __restrict__ P, bf16x4* __restrict__ W1A,
-                           bf16x4* __restrict__ W2A, bf16x4* __restrict__ W2TA) {
-  const int t = threadIdx.x;  // 256 threads: 4 tiles x 64 lanes
+// M[16 row_tile + l % 16][16 k_tile + 4 (l / 16) + e].  t: 0..255, 4 tiles x 64
+// lanes; P: the parameters (global or LDS).
+__device__ __forceinline__ void mlp_pack(int t, const float* P, bf16x4* __restrict__ W1A,
+                                         bf16x4* __restrict__ W2A, bf16x4* __restrict__ W2TA) {
   const int tile = t >> 6, l = t & 63, rt = tile >> 1, kt = tile & 1;
   bf16x4 a, b, c;
 #pragma unroll
@@ -336,6 +385,37 @@ __global__ void k_mlp_pack(const float* __restrict__ P, bf16x4* __restrict__ W1A
   W1A[t] = a;
   W2A[t] = b;
   W2TA[t] = c;
+}
+
+__global__ void k_mlp_pack(const float* __restrict__ P, bf16x4* __restrict__ W1A,
+                           bf16x4* __restrict__ W2A, bf16x4* __restrict__ W2TA) {
+  mlp_pack(threadIdx.x, P, W1A, W2A, W2TA);
+}
+
+// Adam on the fp32 parameters (W1's two padding input columns stay zero) and
+// the operand tiles of the result: one workgroup, so that no second launch has
+// to wait for the first.
+constexpr int ADAM_THREADS = 1024;
+__global__ void __launch_bounds__(ADAM_THREADS) k_mlp_adam(
+    float* __restrict__ P, const float* __restrict__ grad, float* __restrict__ m,
+    float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2,
+    bf16x4* __restrict__ W1A, bf16x4* __restrict__ W2A, bf16x4* __restrict__ W2TA) {
+  __shared__ float Pn[MLP_NPARAM];
+  for (int t = threadIdx.x; t < MLP_NPARAM; t += ADAM_THREADS) {
+    float p = P[t];
+    if (!(t < MLP_B1 && (t % MLP_IN) >= MLP_NFEAT)) {
+      const float g = grad[t];
+      const float mt = b1 * m[t] + (1.0f - b1) * g;
+      const float vt = b2 * v[t] + (1.0f - b2) * g * g;
+      m[t] = mt;
+      v[t] = vt;
+      p -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
+      P[t] = p;
+    }
+    Pn[t] = p;
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) mlp_pack(threadIdx.x, Pn, W1A, W2A, W2TA);
 }
 
 __global__ void k_gather_rows(const float* __restrict__ src, const int64_t* __restrict__ idx,
@@ -416,6 +496,8 @@ struct cbns_mlp {
   float* m = nullptr;
   float* v = nullptr;
   cbns::bf16x4* pack = nullptr;  // 3 x 256 operand tiles
+  float* part = nullptr;         // GRAD_BLOCKS rows of a gradient pass
+  float* host = nullptr;         // pinned: a gradient and its loss, or the parameters
   int t = 0;                     // Adam step count
   std::string err;
 };
@@ -464,6 +546,8 @@ int cbns_mlp_create(cbns_mlp** out) {
       bad(hipMalloc(&m->m, cbns::MLP_NPARAM * sizeof(float))) ||
       bad(hipMalloc(&m->v, cbns::MLP_NPARAM * sizeof(float))) ||
       bad(hipMalloc(&m->pack, 768 * sizeof(cbns::bf16x4))) ||
+      bad(hipMalloc(&m->part, (size_t)cbns::GRAD_BLOCKS * cbns::GRAD_ROW * sizeof(float))) ||
+      bad(hipHostMalloc((void**)&m->host, cbns::GRAD_ROW * sizeof(float), hipHostMallocDefault)) ||
       bad(hipMemset(m->P, 0, cbns::MLP_NPARAM * sizeof(float))) ||
       bad(hipMemset(m->m, 0, cbns::MLP_NPARAM * sizeof(float))) ||
       bad(hipMemset(m->v, 0, cbns::MLP_NPARAM * sizeof(float))))
@@ -479,8 +563,10 @@ int cbns_mlp_create(cbns_mlp** out) {
 void cbns_mlp_destroy(cbns_mlp* m) {
   if (!m) return;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
-  for (void* p : {(void*)m->P, (void*)m->grad, (void*)m->m, (void*)m->v, (void*)m->pack})
+  for (void* p : {(void*)m->P, (void*)m->grad, (void*)m->m, (void*)m->v, (void*)m->pack,
+                  (void*)m->part})
     if (p) (void)hipFree(p);
+  if (m->host) (void)hipHostFree(m->host);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -503,8 +589,10 @@ int cbns_mlp_set_params(cbns_mlp* m, const float* params) {
 
 int cbns_mlp_get_params(cbns_mlp* m, float* params) {
   if (!m || !params) return CBNS_ERR_ARG;
-  MLP_HIP(m, hipMemcpyAsync(params, m->P, cbns::MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+  const size_t nb = cbns::MLP_NPARAM * sizeof(float);
+  MLP_HIP(m, hipMemcpyAsync(m->host, m->P, nb, hipMemcpyDeviceToHost, m->stream));
   MLP_HIP(m, hipStreamSynchronize(m->stream));
+  std::memcpy(params, m->host, nb);
   return CBNS_OK;
 }
 
@@ -522,21 +610,21 @@ int cbns_mlp_forward(cbns_mlp* m, const float* feat, int64_t n, float* logit) {
 int cbns_mlp_loss_grad(cbns_mlp* m, const float* feat, const float* target, int64_t n, float w_pos,
                        double* loss, float* grad) {
   if (!m || n <= 0 || !feat || !target) return CBNS_ERR_ARG;
-  const long chunks = (n + 63) / 64;
-  const long waves = std::min<long>(chunks, 4L * 1024);
-  const unsigned blocks = (unsigned)((waves + 3) / 4);
-  const int iters = (int)((chunks + 4L * blocks - 1) / (4L * blocks));
-  MLP_HIP(m, hipMemsetAsync(m->grad, 0, (cbns::MLP_NPARAM + 1) * sizeof(float), m->stream));
-  cbns::k_mlp_grad<<<blocks, 256, 0, m->stream>>>(mlp_dev(m), feat, target, n, w_pos,
-                                                  1.0f / (float)n, iters, m->grad,
-                                                  m->grad + cbns::MLP_NPARAM);
+  const long tiles = (n + 15) / 16;
+  const int blocks = (int)std::min<long>((tiles + cbns::GRAD_WAVES - 1) / cbns::GRAD_WAVES,
+                                         cbns::GRAD_BLOCKS);
+  const long per_it = (long)blocks * cbns::GRAD_WAVES;
+  const int iters = (int)((tiles + per_it - 1) / per_it);
+  cbns::k_mlp_grad<<<blocks, 64 * cbns::GRAD_WAVES, 0, m->stream>>>(
+      mlp_dev(m), feat, target, n, w_pos, 1.0f / (float)n, iters, m->part);
   MLP_HIP(m, hipGetLastError());
-  float lsum = 0.0f;
-  MLP_HIP(m, hipMemcpyAsync(&lsum, m->grad + cbns::MLP_NPARAM, sizeof(float), hipMemcpyDeviceToHost, m->stream));
-  if (grad)
-    MLP_HIP(m, hipMemcpyAsync(grad, m->grad, cbns::MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+  // the sums reach the host as the last pass writes them
+  cbns::k_mlp_sum<<<(cbns::MLP_NPARAM + 1 + 63) / 64, 64 * cbns::SUM_WAVES, 0, m->stream>>>(
+      m->part, blocks, m->grad, m->host);
+  MLP_HIP(m, hipGetLastError());
   MLP_HIP(m, hipStreamSynchronize(m->stream));
-  if (loss) *loss = (double)lsum / (double)n;
+  if (grad) std::memcpy(grad, m->host, cbns::MLP_NPARAM * sizeof(float));
+  if (loss) *loss = (double)m->host[cbns::MLP_NPARAM] / (double)n;
   return CBNS_OK;
 }
 
@@ -545,10 +633,10 @@ int cbns_mlp_adam_step(cbns_mlp* m, float lr, float beta1, float beta2, float ep
   m->t++;
   const float c1 = (float)(1.0 - std::pow((double)beta1, m->t));
   const float c2 = (float)(1.0 - std::pow((double)beta2, m->t));
-  cbns::k_mlp_adam<<<(cbns::MLP_NPARAM + 255) / 256, 256, 0, m->stream>>>(m->P, m->grad, m->m, m->v,
-                                                                          lr, beta1, beta2, eps, c1, c2);
+  cbns::k_mlp_adam<<<1, cbns::ADAM_THREADS, 0, m->stream>>>(m->P, m->grad, m->m, m->v, lr, beta1,
+                                                            beta2, eps, c1, c2, m->pack,
+                                                            m->pack + 256, m->pack + 512);
   MLP_HIP(m, hipGetLastError());
-  if (int rc = mlp_repack(m)) return rc;
   MLP_HIP(m, hipStreamSynchronize(m->stream));
   return CBNS_OK;
 }
