@@ -71,7 +71,7 @@ EXPORTS = [
     "cbns_get_primitive", "cbns_set_bc_calc_primitive", "cbns_calc_dt",
     "cbns_calc_numerical_flux", "cbns_calc_viscous_terms",
     "cbns_calc_viscous_flux_contribution", "cbns_update_rk3", "cbns_rk3_stage",
-    "cbns_rk3_step", "cbns_set_form", "cbns_get_field", "cbns_set_field",
+    "cbns_rk3_step", "cbns_set_form", "cbns_get_field", "cbns_get_fields", "cbns_set_field",
     "cbns_synchronize", "cbns_field_size", "cbns_set_profiling", "cbns_kernel_time",
     "cbns_face_count", "cbns_face_samples", "cbns_set_indicator", "cbns_flag_count",
     "cbns_get_flags", "cbns_dev_alloc", "cbns_dev_free", "cbns_dev_upload", "cbns_dev_download",
@@ -119,6 +119,7 @@ def lib():
         "cbns_rk3_step": ([B, C.c_double, D, D], C.c_int),
         "cbns_set_form": ([B, I], C.c_int),
         "cbns_get_field": ([B, I, D], C.c_int),
+        "cbns_get_fields": ([B, I, I, D], C.c_int),
         "cbns_set_field": ([B, I, D], C.c_int),
         "cbns_synchronize": ([B], C.c_int),
         "cbns_field_size": ([B], C.c_int64),
@@ -280,8 +281,7 @@ class Block:
     # -- raw ghosted SoA fields ---------------------------------------------
     def get_field(self, f, n=1):
         out = np.zeros((n,) + self.shape)
-        for q in range(n):
-            self._chk(lib().cbns_get_field(self._h, f + q, _ptr(out[q])))
+        self._chk(lib().cbns_get_fields(self._h, f, n, _ptr(out)))
         return out if n > 1 else out[0]
 
     def set_field(self, f, arr):

@@ -90,6 +90,14 @@ double* field_ptr(cbns_block* b, int f) {
   return nullptr;
 }
 
+// fields from f to the end of the array that holds it
+int fields_left(int f) {
+  for (const auto& [first, n] : {std::pair{CBNS_F_Q, 5}, {CBNS_F_QP, 5}, {CBNS_F_PRIM, 6},
+                                 {CBNS_F_MET, 10}, {CBNS_F_FLUX, 15}, {CBNS_F_DFV, 4}})
+    if (f >= first && f < first + n) return first + n - f;
+  return 1;
+}
+
 // copy between a 2-ghost-layer host array (the reference's IM_G x JM_G x KM_G
 // layout, src/Block3d.cpp:325-335) and one device field
 void ref_to_internal(const Consts& c, const double* src, long src_stride, long src_off,
@@ -177,7 +185,10 @@ int cbns_create(const cbns_params* p, cbns_block** out) {
   if (!b) return CBNS_ERR_ARG;
   b->p = *p;
   derive(b);
+  host_copy_ref();
+  b->copy_ref = true;
   if (hipGetDevice(&b->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess) {
+    host_copy_unref();
     delete b;
     return CBNS_ERR_HIP;
   }
@@ -234,6 +245,7 @@ void cbns_destroy(cbns_block* b) {
     (void)hipEventDestroy(ev.second);
   }
   if (b->stream) (void)hipStreamDestroy(b->stream);
+  if (b->copy_ref) host_copy_unref();
   delete b;
 }
 
@@ -581,14 +593,21 @@ int cbns_flag_count(cbns_block* b, int64_t counts[3]) {
   return CBNS_OK;
 }
 
-int cbns_get_field(cbns_block* b, int32_t f, double* host) {
-  if (!b || !host) return CBNS_ERR_ARG;
+int cbns_get_field(cbns_block* b, int32_t f, double* host) { return cbns_get_fields(b, f, 1, host); }
+
+int cbns_get_fields(cbns_block* b, int32_t f, int32_t n, double* host) {
+  if (!b || !host || n < 0) return CBNS_ERR_ARG;
   CBNS_HIP(b, hipSetDevice(b->device));
-  if (f >= CBNS_F_FLUX && ensure_unfused(b)) return CBNS_ERR_HIP;
-  double* d = field_ptr(b, f);
-  if (!d) return fail(b, CBNS_ERR_ARG, "field not available");
-  CBNS_HIP(b, hipMemcpyAsync(host, d, sizeof(double) * b->c.S, hipMemcpyDeviceToHost, b->stream));
-  CBNS_HIP(b, hipStreamSynchronize(b->stream));
+  for (long S = b->c.S; n > 0;) {
+    if (f >= CBNS_F_FLUX && ensure_unfused(b)) return CBNS_ERR_HIP;
+    const double* d = field_ptr(b, f);
+    if (!d) return fail(b, CBNS_ERR_ARG, "field not available");
+    const int m = std::min(n, fields_left(f));  // one array, one copy
+    if (int rc = copy_to_host(b, d, host, sizeof(double) * m * S)) return rc;
+    host += m * S;
+    f += m;
+    n -= m;
+  }
   return CBNS_OK;
 }
 

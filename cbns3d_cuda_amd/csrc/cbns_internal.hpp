@@ -301,6 +301,7 @@ struct cbns_block {
   long toff[3] = {0, 0, 0};      // first slot of each axis
   long ttotal = 0;               // slots in all (tflux's field stride)
   bool tfull = false;            // a list overflowed: the marches run WENO at every face
+  bool copy_ref = false;         // holds a reference to host_copy.hip's staging
   std::string err;
 };
 
@@ -367,6 +368,11 @@ int launch_dt_device(cbns_block* b, double cap, double* out);
 int launch_sutherland(cbns_block* b);
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout);
 int launch_fill(hipStream_t s, double* p, long n, double v);
+// device memory into a caller's host memory, complete on return (host_copy.hip);
+// each block holds a reference to the copies' shared staging
+int copy_to_host(cbns_block* b, const void* dev, void* host, size_t bytes);
+void host_copy_ref();
+void host_copy_unref();
 long face_count(const cbns_block* b, int axis);
 int launch_face_samples(cbns_block* b, int axis, const double* Q, float* feat, float* label);
 int launch_indicator(cbns_block* b, const double* Q);

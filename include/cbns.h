@@ -152,6 +152,8 @@ int cbns_set_form(cbns_block* blk, int32_t form);
 
 /* raw ghosted SoA field access (tests, tools) */
 int cbns_get_field(cbns_block* blk, int32_t field, double* host);
+/* fields field .. field + n - 1, one after another */
+int cbns_get_fields(cbns_block* blk, int32_t field, int32_t n, double* host);
 int cbns_set_field(cbns_block* blk, int32_t field, const double* host);
 int cbns_synchronize(cbns_block* blk);
 /* doubles per ghosted field, (IM+2G)*(JM+2G)*(KM+2G) */
