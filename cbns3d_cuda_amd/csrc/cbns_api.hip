@@ -459,6 +459,7 @@ int cbns_rk3_stage(cbns_block* b, double dt, int32_t stage) {
   double* qout = stage == 1 ? b->qp : (stage == 2 ? b->qspare : b->Q);
   if ((rc = launch_fused_stage(b, dt, stage, qin, qout))) return rc;
   if (stage == 2) std::swap(b->qp, b->qspare);
+  if (stage_wraps(b->c, dt)) return CBNS_OK;
   ProfScope ps(b, CBNS_K_BC);
   return launch_bc_only(b, stage == 3 ? b->Q : b->qp, stage_prim_mask(b, stage));
 }
@@ -489,7 +490,19 @@ int cbns_rk3_step(cbns_block* b, double t_end, double* t_cur, double* dt_out) {
                              hipMemcpyDeviceToHost, b->stream));
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   const double dt = b->h_scalar[2];
-  if (std::isnan(dt)) return fail(b, CBNS_ERR_NAN, "An error occurred while calculating the time step.");
+  if (std::isnan(dt)) {
+    // the marches left the stages' outputs as they were; so are their ghosts
+    // filled as a stage would
+    if (stage_wraps(b->c, 0.0)) {
+      b->step_internal = true;
+      if (!(rc = launch_bc_only(b, b->qspare, stage_prim_mask(b, 1))) &&
+          !(rc = launch_bc_only(b, b->qp, stage_prim_mask(b, 2))))
+        rc = launch_bc_only(b, b->Q, stage_prim_mask(b, 3));
+      b->step_internal = false;
+      if (rc) return rc;
+    }
+    return fail(b, CBNS_ERR_NAN, "An error occurred while calculating the time step.");
+  }
   *t_cur += dt;
   if (dt_out) *dt_out = dt;
   return CBNS_OK;

@@ -346,6 +346,18 @@ inline int stage_prim_mask(const cbns_block* b, int stage) {
   const int pall = b->c.viscous ? 0x3F : 0x1F;
   return b->step_internal && stage < 3 ? (b->c.viscous ? 0x2E : 0) : pall;
 }
+// The stage's last march writes the ghosts with the state where every axis is
+// periodic, no node reaches the ghosts of both ends and the block is small: a
+// launch less against stores of partial lines that its wavefronts wait for.
+// Step, us, fill launch / march (FP64): inviscid 24^3 93 / 85, 48^3 136 / 136,
+// 96^3 487 / 516; viscous 24^3 121 / 113, 48^3 185 / 182, 64^3 276 / 278, 96^3
+// 710 / 748; the float and hybrid forms cross between 64^3 and 80^3.  (S counts
+// ghosts: 2^18 is 56^3 nodes.)  A time step known to be NaN leaves the state,
+// and its ghosts to the fill.
+inline bool stage_wraps(const Consts& c, double dt) {
+  return periodic(c, 0) && periodic(c, 1) && periodic(c, 2) && c.IM >= 2 * G && c.JM >= 2 * G &&
+         c.KM >= 2 * G && c.S <= 1 << 18 && dt == dt;
+}
 int launch_primitive_all(cbns_block* b, const double* Q);
 int launch_conservative_all(cbns_block* b, double* Q);
 int launch_freestream(cbns_block* b);

@@ -130,8 +130,8 @@ struct StageArgs {
 };
 
 // AX = 1: march along eta, rhs = dF.  AX = 2: march along zeta with the
-// xi-faces, finish.
-template <int AX, class F, bool HYB>
+// xi-faces, finish; WRAP: and write the periodic ghosts (stage_wraps).
+template <int AX, class F, bool HYB, bool WRAP>
 __global__ void __launch_bounds__(MARCH_X * MARCH_Y)
 __attribute__((amdgpu_waves_per_eu(HYB ? WPE_H : WPE_M, HYB ? WPE_H : WPE_M)))
 k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
@@ -462,19 +462,39 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
         if (sa.stage == 1) out = qin - dt * df;
         else if (sa.stage == 2) out = 0.75 * qnv[n] + 0.25 * (qin - dt * df);
         else out = (qnv[n] + 2.0 * (qin - dt * df)) * (1.0 / 3.0);
-        if (own) sa.Qout[n * S + o] = out;
         qn_out[n] = out;
       }
       // primitives of the new state (src/primitive_bc_kernel.cu:63-76)
       if (own) {
         double rr, uu, vv, ww, pp;
         q_to_prim(g, qn_out, rr, uu, vv, ww, pp);
-        if (sa.pmask & 1) sa.prim[o] = rr;
-        if (sa.pmask & 2) sa.prim[S + o] = uu;
-        if (sa.pmask & 4) sa.prim[2 * S + o] = vv;
-        if (sa.pmask & 8) sa.prim[3 * S + o] = ww;
-        if (sa.pmask & 16) sa.prim[4 * S + o] = pp;
-        if (sa.pmask & 32) sa.prim[5 * S + o] = c.gM2 * pp * fast_rcp(rr);
+        const double tt = c.gM2 * pp * fast_rcp(rr);
+        const auto put = [&](int d) {
+#pragma unroll
+          for (int n = 0; n < 5; n++) sa.Qout[n * S + d] = qn_out[n];
+          if (sa.pmask & 1) sa.prim[d] = rr;
+          if (sa.pmask & 2) sa.prim[S + d] = uu;
+          if (sa.pmask & 4) sa.prim[2 * S + d] = vv;
+          if (sa.pmask & 8) sa.prim[3 * S + d] = ww;
+          if (sa.pmask & 16) sa.prim[4 * S + d] = pp;
+          if (sa.pmask & 32) sa.prim[5 * S + d] = tt;
+        };
+        put(o);
+        if constexpr (WRAP) {
+          // the node's images in the ghosts: along each axis at whose end it
+          // lies, and along each pair and all three of them
+          const int di = i < G ? c.IM : (i >= c.IM - G ? -c.IM : 0);
+          const int dj = t < G ? c.JM : (t >= c.JM - G ? -c.JM : 0);
+          const int dk = m < G ? c.KM : (m >= c.KM - G ? -c.KM : 0);
+          if (di | dj | dk) {
+#pragma unroll 1
+            for (int im = 1; im < 8; im++) {
+              const int ex = im & 1 ? di : 0, ey = im & 2 ? dj : 0, ez = im & 4 ? dk : 0;
+              if ((im & 1 && !ex) || (im & 2 && !ey) || (im & 4 && !ez)) continue;
+              put(o + ex + ey * c.PX + ez * c.PXY);
+            }
+          }
+        }
       }
     }
 #pragma unroll
@@ -667,7 +687,7 @@ static MarchCut march_cut(long lines, int n) {
   return best;
 }
 
-template <int AX, class F, bool HYB>
+template <int AX, class F, bool HYB, bool WRAP = false>
 int launch_march(cbns_block* b, StageArgs& sa) {
   const Consts& c = b->c;
   const int ax_t = AX == 1 ? 2 : 1;
@@ -683,7 +703,7 @@ int launch_march(cbns_block* b, StageArgs& sa) {
   const int R = cut.waves <= 1024 ? 1 : MARCH_Y;
   const dim3 grid((unsigned)((nw + R - 1) / R), sa.parts, (nm + CHUNK_MAX - 1) / CHUNK_MAX);
   ProfScope ps(b, AX == 1 ? CBNS_K_MARCH_ETA : CBNS_K_MARCH_ZETA);
-  k_march<AX, F, HYB><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
+  k_march<AX, F, HYB, WRAP><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
 }
@@ -744,6 +764,8 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
     sa.flags = fl + 2 * S;
     sa.tf.slot = b->tslot + 2 * S;
   }
+  if (stage_wraps(c, dt))
+    return hyb ? launch_march<2, F, true, true>(b, sa) : launch_march<2, F, false, true>(b, sa);
   return hyb ? launch_march<2, F, true>(b, sa) : launch_march<2, F, false>(b, sa);
 }
 
