@@ -116,7 +116,10 @@ template <class T>
 __device__ __forceinline__ void roe_basis_q(const GasT<T>& g, const T qL[5], const T qR[5],
                                             T n_x, T n_y, T n_z, Basis<T>& B) {
   const T aL = fast_rsq(qL[0]), aR = fast_rsq(qR[0]);
-  const T D = fast_rcp(qL[0] * aL + qR[0] * aR);
+  // the left product named: the zeta march shares it between the faces that
+  // leave a node, and which of the two the compiler fuses would follow the code
+  // around it
+  const T D = fast_rcp(fma(qR[0], aR, qL[0] * aL));
   const T wL = aL * D, wR = aR * D;
   // p = gam1 (E - |rho u|^2 / (2 rho)), 1/rho = a^2
   const T pL = g.gam1 * (qL[4] - T(0.5) * (qL[1] * qL[1] + qL[2] * qL[2] + qL[3] * qL[3]) * (aL * aL));

@@ -127,11 +127,14 @@ struct StageArgs {
   TroubledFaces tf;     // WENO fluxes of the march axis' troubled faces (HYB)
   TroubledFaces tf_x;   // and of the troubled xi-faces (HYB, AX == 2)
   int parts;            // chunks per CHUNK_MAX nodes of a line
+  bool wrap;            // AX == 2, SHORT: write the periodic ghosts too (stage_wraps)
 };
 
 // AX = 1: march along eta, rhs = dF.  AX = 2: march along zeta with the
-// xi-faces, finish; WRAP: and write the periodic ghosts (stage_wraps).
-template <int AX, class F, bool HYB, bool WRAP>
+// xi-faces, finish.  SHORT (zeta): the march of short chunks, whose first pass
+// leaves out the xi-faces that it does not use, and which can write the
+// periodic ghosts.
+template <int AX, class F, bool HYB, bool SHORT>
 __global__ void __launch_bounds__(MARCH_X * MARCH_Y)
 __attribute__((amdgpu_waves_per_eu(HYB ? WPE_H : WPE_M, HYB ? WPE_H : WPE_M)))
 k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
@@ -333,7 +336,7 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
       xmy = met[XI_Y * S + o];
       xmz = met[XI_Z * S + o];
     }
-    if constexpr (XI) {
+    if (XI && (!SHORT || upd)) {
       // the xi-face between node (i, m) and (i+1, m): stencil i-2 .. i+3
       // (every lane takes part in the shuffles)
       double qx[6][5];
@@ -469,6 +472,9 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
         double rr, uu, vv, ww, pp;
         q_to_prim(g, qn_out, rr, uu, vv, ww, pp);
         const double tt = c.gM2 * pp * fast_rcp(rr);
+        // all stores of a node together, after its arithmetic: with the state's
+        // ahead of the primitives 256^3 took 1610 us for 1531 (hybrid 1203 for
+        // 1165)
         const auto put = [&](int d) {
 #pragma unroll
           for (int n = 0; n < 5; n++) sa.Qout[n * S + d] = qn_out[n];
@@ -480,7 +486,7 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
           if (sa.pmask & 32) sa.prim[5 * S + d] = tt;
         };
         put(o);
-        if constexpr (WRAP) {
+        if (SHORT && sa.wrap) {
           // the node's images in the ghosts: along each axis at whose end it
           // lies, and along each pair and all three of them
           const int di = i < G ? c.IM : (i >= c.IM - G ? -c.IM : 0);
@@ -666,6 +672,11 @@ struct MarchCut {
   int parts;   // chunks per CHUNK_MAX nodes
   long waves;  // wavefronts in all
 };
+// Chunks of up to CHUNK_MAX / PARTS_SHORT nodes skip the xi-faces of their first
+// pass by a branch: 64^3 zeta march 41.5 -> 38.5 us.  In long ones the branch
+// parts the arithmetic of the two faces for little: 256^3 1531 us, 1570 with it.
+// From 8 to 16 nodes a chunk both are within the noise.
+constexpr int PARTS_SHORT = 4;
 static MarchCut march_cut(long lines, int n) {
   constexpr long SLOTS = 2048;
   constexpr double PAIR = 1.8;
@@ -687,7 +698,7 @@ static MarchCut march_cut(long lines, int n) {
   return best;
 }
 
-template <int AX, class F, bool HYB, bool WRAP = false>
+template <int AX, class F, bool HYB>
 int launch_march(cbns_block* b, StageArgs& sa) {
   const Consts& c = b->c;
   const int ax_t = AX == 1 ? 2 : 1;
@@ -703,7 +714,9 @@ int launch_march(cbns_block* b, StageArgs& sa) {
   const int R = cut.waves <= 1024 ? 1 : MARCH_Y;
   const dim3 grid((unsigned)((nw + R - 1) / R), sa.parts, (nm + CHUNK_MAX - 1) / CHUNK_MAX);
   ProfScope ps(b, AX == 1 ? CBNS_K_MARCH_ETA : CBNS_K_MARCH_ZETA);
-  k_march<AX, F, HYB, WRAP><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
+  const bool brief = AX == 2 && (sa.parts >= PARTS_SHORT || sa.wrap);
+  const auto kern = brief ? k_march<AX, F, HYB, AX == 2> : k_march<AX, F, HYB, false>;
+  kern<<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
 }
@@ -752,7 +765,7 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
                b->rhs, c.viscous ? b->vtmp : nullptr,
                hyb ? fl + S : nullptr, hyb ? fl : nullptr, pmask,
                TroubledFaces{hyb ? b->tslot + S : nullptr, b->tflux, b->ttotal},
-               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1};
+               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1, stage_wraps(c, dt)};
   if ((rc = hyb ? launch_march<1, F, true>(b, sa) : launch_march<1, F, false>(b, sa)))
     return rc;
   if (lam) {
@@ -764,8 +777,6 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
     sa.flags = fl + 2 * S;
     sa.tf.slot = b->tslot + 2 * S;
   }
-  if (stage_wraps(c, dt))
-    return hyb ? launch_march<2, F, true, true>(b, sa) : launch_march<2, F, false, true>(b, sa);
   return hyb ? launch_march<2, F, true>(b, sa) : launch_march<2, F, false>(b, sa);
 }
 
