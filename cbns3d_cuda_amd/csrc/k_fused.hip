@@ -86,7 +86,20 @@ struct TroubledFaces {
 // transverse indices; 0 for the centred divergence).
 template <class T>
 __device__ __forceinline__ T visc_face(T vm1, T v0, T v1, T v2) {
-  return T(7.0 / 12.0) * (v0 + v1) - T(1.0 / 12.0) * (vm1 + v2);
+  return fma(T(7.0 / 12.0), v0 + v1, -(T(1.0 / 12.0) * (vm1 + v2)));
+}
+
+// J grad xi of a face, from J and a metric term of its two nodes: the plain form
+// rounds both products, the others node m+1's (LEFT) or node m's.
+enum Rounding { BOTH, LEFT, RIGHT };
+template <class F, bool HYB>
+constexpr Rounding rounding(bool left) {
+  return sizeof(F) == sizeof(double) && !HYB ? BOTH : (left ? LEFT : RIGHT);
+}
+__device__ __forceinline__ double face_normal(Rounding r, double m0, double j0, double m1,
+                                              double j1) {
+  return 0.5 * (r == BOTH ? m0 * j0 + m1 * j1
+                          : (r == LEFT ? fma(m0, j0, m1 * j1) : fma(m1, j1, m0 * j0)));
 }
 
 // Face flux of the stage's form at face `face` (node offset).  HYB: the
@@ -98,9 +111,19 @@ __device__ __forceinline__ T visc_face(T vm1, T v0, T v1, T v2) {
 template <class F, bool HYB>
 __device__ __forceinline__ void stage_face(const GasT<double>& g, const double q[6][5],
                                            double nx, double ny, double nz, bool troubled,
-                                           const TroubledFaces& tf, int face, double f[5]) {
-  if (!HYB) {
-    face_flux_form<F>(g, q, nx, ny, nz, f);
+                                           const TroubledFaces& tf, int face, bool yz,
+                                           double f[5]) {
+  if constexpr (!HYB) {
+    F e[5][5];
+    stencil_diffs(q, e);
+    if constexpr (sizeof(F) == sizeof(double)) {
+      face_flux(g, e, q[2], q[3], nx, ny, nz, f);
+    } else {
+      F d[6][5];
+      dev_from_diffs(e, d);
+      face_flux_dev<true>(g, d, q[2], node_t<F>(g, q_to_side(g, q[2])), node_t<F>(g, q_to_side(g, q[3])),
+                    nx, ny, nz, yz, f);
+    }
     return;
   }
   face_linear<F>(g, q, nx, ny, nz, f);
@@ -127,14 +150,66 @@ struct StageArgs {
   TroubledFaces tf;     // WENO fluxes of the march axis' troubled faces (HYB)
   TroubledFaces tf_x;   // and of the troubled xi-faces (HYB, AX == 2)
   int parts;            // chunks per CHUNK_MAX nodes of a line
-  bool wrap;            // AX == 2, SHORT: write the periodic ghosts too (stage_wraps)
 };
 
+// The Shu-Osher combination of node o = (i, j, k) from its flux differences
+// along xi (de), eta (df) and zeta (dg), its state qin, level-n state qn and
+// Jacobian; with `own` also its stores.  WRAP: the periodic ghosts too.
+template <bool WRAP>
+__device__ __forceinline__ void finish_node(const Consts& c, const StageArgs& sa,
+                                            const GasT<double>& g, double dt, int i, int j, int k,
+                                            int o, bool own, const double de[5],
+                                            const double df[5], const double dg[5],
+                                            const double qin[5], const double qn[5], double jac) {
+  const long S = c.S;
+  const double inv_j = fast_rcp(jac);
+  double out[5];
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    const double euler = fma(-dt, (df[n] + dg[n] + de[n]) * inv_j, qin[n]);
+    if (sa.stage == 1) out[n] = euler;
+    else if (sa.stage == 2) out[n] = fma(0.25, euler, 0.75 * qn[n]);
+    else out[n] = fma(2.0, euler, qn[n]) * (1.0 / 3.0);
+  }
+  if (!own) return;
+  // primitives of the new state (src/primitive_bc_kernel.cu:63-76)
+  double rr, uu, vv, ww, pp;
+  q_to_prim(g, out, rr, uu, vv, ww, pp);
+  const double tt = c.gM2 * pp * fast_rcp(rr);
+  // all stores of a node together, after its arithmetic: with the state's
+  // ahead of the primitives the 256^3 zeta march took 1610 us for 1531 (hybrid
+  // 1203 for 1165)
+  const auto put = [&](int d) {
+#pragma unroll
+    for (int n = 0; n < 5; n++) sa.Qout[n * S + d] = out[n];
+    if (sa.pmask & 1) sa.prim[d] = rr;
+    if (sa.pmask & 2) sa.prim[S + d] = uu;
+    if (sa.pmask & 4) sa.prim[2 * S + d] = vv;
+    if (sa.pmask & 8) sa.prim[3 * S + d] = ww;
+    if (sa.pmask & 16) sa.prim[4 * S + d] = pp;
+    if (sa.pmask & 32) sa.prim[5 * S + d] = tt;
+  };
+  put(o);
+  if (WRAP) {
+    // the node's images in the ghosts: along each axis at whose end it
+    // lies, and along each pair and all three of them
+    const int di = i < G ? c.IM : (i >= c.IM - G ? -c.IM : 0);
+    const int dj = j < G ? c.JM : (j >= c.JM - G ? -c.JM : 0);
+    const int dk = k < G ? c.KM : (k >= c.KM - G ? -c.KM : 0);
+    if (di | dj | dk) {
+#pragma unroll 1
+      for (int im = 1; im < 8; im++) {
+        const int ex = im & 1 ? di : 0, ey = im & 2 ? dj : 0, ez = im & 4 ? dk : 0;
+        if ((im & 1 && !ex) || (im & 2 && !ey) || (im & 4 && !ez)) continue;
+        put(o + ex + ey * c.PX + ez * c.PXY);
+      }
+    }
+  }
+}
+
 // AX = 1: march along eta, rhs = dF.  AX = 2: march along zeta with the
-// xi-faces, finish.  SHORT (zeta): the march of short chunks, whose first pass
-// leaves out the xi-faces that it does not use, and which can write the
-// periodic ghosts.
-template <int AX, class F, bool HYB, bool SHORT>
+// xi-faces, finish.  WRAP (zeta): also writes the periodic ghosts (stage_wraps).
+template <int AX, class F, bool HYB, bool WRAP>
 __global__ void __launch_bounds__(MARCH_X * MARCH_Y)
 __attribute__((amdgpu_waves_per_eu(HYB ? WPE_H : WPE_M, HYB ? WPE_H : WPE_M)))
 k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
@@ -172,39 +247,34 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
   const double* __restrict__ J = met + JAC * S;
   const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
 
-  // The face left of the chunk's first node.  Where CHUNK_MAX nodes of the
-  // line have passed (head) it is formed here, ahead of the loop; elsewhere by
-  // a first pass of the loop (m = m0 - 1) that forms the faces only.  The
-  // compiler fuses products otherwise here than in the loop, so with this rule
-  // a line's faces are those of chunks of CHUNK_MAX nodes, bit for bit,
-  // whatever the chunk: a last bit, rounded to float in the precision form or
-  // fed to the hybrid's indicator, can move a flux by a float's last bit of a
-  // shock's jump or flip a troubled flag.
-  const bool head = part == 0;
-  const int mb = head ? m0 : m0 - 1;  // first pass of the loop
   double q[6][5];  // nodes m-2 .. m+3 for the face m+1/2, of the pass before
 #pragma unroll
-  for (int s = 0; s < 6; s++) load_q(Q, S, base + (mb - 3 + s) * st, q[s]);
+  for (int s = 0; s < 6; s++) load_q(Q, S, base + (m0 - 3 + s) * st, q[s]);
   // J grad xi_AX at the face's two nodes
-  int o = base + (mb - 1) * st;
+  int o = base + (m0 - 1) * st;
   double jb = J[o + st];
-  double ax = 0.0, ay = 0.0, az = 0.0;
-  double bx = nX[o + st] * jb, by = nY[o + st] * jb, bz = nZ[o + st] * jb;
-  double fprev[5] = {0, 0, 0, 0, 0};
+  // metric terms of the face's right node; where both products of a face normal
+  // are rounded, with J, since they are the next face's left ones
+  constexpr bool PROD = rounding<F, HYB>(false) == BOTH;
+  double mx = nX[o + st], my = nY[o + st], mz = nZ[o + st];
+  if (PROD) { mx *= jb; my *= jb; mz *= jb; }
+  const auto normal = [&](Rounding r, double a, double ja, double m, double jm) {
+    return PROD ? 0.5 * (a + m) : face_normal(r, a, ja, m, jm);
+  };
+  double fprev[5];
   // troubled flags of faces m-1, m, m+1 (face m between nodes m and m+1)
   const uint8_t* __restrict__ fl = sa.flags;
   uint8_t t0 = 0, t1 = 0, t2 = 0;
   if (HYB) {
-    t0 = fl[base + (mb - 2) * st];
-    t1 = fl[base + (mb - 1) * st];
-    t2 = fl[base + mb * st];
+    t0 = fl[base + (m0 - 2) * st];
+    t1 = fl[base + (m0 - 1) * st];
+    t2 = fl[base + m0 * st];
   }
   // Precision form (float faces, not hybrid): the sweep carries the float
   // differences e[k] = q[k+1] - q[k] of the window's nodes and the Roe
   // inputs of nodes m (nl) and m+1 (nr), each formed once per node, instead
   // of five double differences and two double face states per face.
   constexpr bool DC = sizeof(F) != sizeof(double) && !HYB;
-  const GasT<F> gt{(F)c.gamma, (F)c.gam1, (F)c.gam1_inv};
   F e[5][5];
   NodeT<F> nl{}, nr{};
   if constexpr (DC) {
@@ -215,17 +285,23 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
     nl = node_t<F>(g, q_to_side(g, q[2]));
     nr = node_t<F>(g, q_to_side(g, q[3]));
   }
-  if (head) {
+  // the face left of the chunk's first node
+  {
     const double ja = J[o];
-    ax = nX[o] * ja; ay = nY[o] * ja; az = nZ[o] * ja;
+    double ax = nX[o], ay = nY[o], az = nZ[o];
+    if (PROD) { ax *= ja; ay *= ja; az *= ja; }
+    // (the first of a line's CHUNK_MAX nodes rounds the other product)
+    const bool first = part == 0;
+    const Rounding r = rounding<F, HYB>(first);
+    const double sx = normal(r, ax, ja, mx, jb), sy = normal(r, ay, ja, my, jb);
+    const double sz = normal(r, az, ja, mz, jb);
     if constexpr (DC) {
       F d[6][5];
       dev_from_diffs(e, d);
-      face_flux_dev<F>(gt, g, d, q[2], nl, nr, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz),
-                       fprev);
+      face_flux_dev<true>(g, d, q[2], nl, nr, sx, sy, sz, AX == 1 && !first, fprev);
     } else {
-      stage_face<F, HYB>(g, q, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz), t0 | t1 | t2,
-                         sa.tf, o, fprev);
+      stage_face<F, HYB>(g, q, sx, sy, sz, t0 | t1 | t2, sa.tf, o, AX == 1 && !first,
+                         fprev);
     }
   }
   // viscous node flux of the march axis (Fv or Gv) on its offset line,
@@ -252,8 +328,8 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
     for (int e = 0; e < 4; e++) {
       F w[4];
 #pragma unroll
-      for (int s = 0; s < 4; s++) w[s] = va[e * S + vbase + (mb - 2 + s) * st];
-      if (head) fprev[e + 1] -= (double)visc_face(w[0], w[1], w[2], w[3]);
+      for (int s = 0; s < 4; s++) w[s] = va[e * S + vbase + (m0 - 2 + s) * st];
+      fprev[e + 1] -= (double)visc_face(w[0], w[1], w[2], w[3]);
 #pragma unroll
       for (int s = 0; s < 3; s++) {
         if constexpr (VRING) vring[s][e][ty][tl] = w[s + 1];
@@ -268,12 +344,11 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
   constexpr bool PF = AX == 1 && !HYB;
   double qpf[5] = {0, 0, 0, 0, 0}, jpf = 0.0, xpf = 0.0, ypf = 0.0, zpf = 0.0;
   if constexpr (PF) {
-    load_q(Q, S, base + (mb + 3) * st, qpf);
-    const int on = base + (mb + 1) * st;
+    load_q(Q, S, base + (m0 + 3) * st, qpf);
+    const int on = base + (m0 + 1) * st;
     jpf = J[on]; xpf = nX[on]; ypf = nY[on]; zpf = nZ[on];
   }
-  for (int m = mb; m < m1; m++) {
-    const bool upd = m >= m0;  // false in the first pass
+  for (int m = m0; m < m1; m++) {
     // shift the window by one node
 #pragma unroll
     for (int s = 0; s < 5; s++)
@@ -319,16 +394,17 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
         qnv[n] = sa.stage > 1 ? sa.Qn[n * S + o] : 0.0;
       }
     }
-    ax = bx; ay = by; az = bz;
+    const double ax = mx, ay = my, az = mz;
     if constexpr (PF) {
       jb = jpf;
-      bx = xpf * jb; by = ypf * jb; bz = zpf * jb;
+      mx = xpf; my = ypf; mz = zpf;
       const int on = o + 2 * st;
       jpf = J[on]; xpf = nX[on]; ypf = nY[on]; zpf = nZ[on];
     } else {
       jb = J[o + st];
-      bx = nX[o + st] * jb; by = nY[o + st] * jb; bz = nZ[o + st] * jb;
+      mx = nX[o + st]; my = nY[o + st]; mz = nZ[o + st];
     }
+    if (PROD) { mx *= jb; my *= jb; mz *= jb; }
     double f[5], fxr[5];
     double xmx = 0.0, xmy = 0.0, xmz = 0.0;  // xi metrics of node m
     if (XI) {
@@ -336,10 +412,10 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
       xmy = met[XI_Y * S + o];
       xmz = met[XI_Z * S + o];
     }
-    if (XI && (!SHORT || upd)) {
+    if (XI) {
       // the xi-face between node (i, m) and (i+1, m): stencil i-2 .. i+3
       // (every lane takes part in the shuffles)
-      double qx[6][5];
+      double qx[2][5];
       if constexpr (HYB) {
         // linear xi-face from the neighbouring lanes' values, one
         // component at a time (six values live, not the whole stencil)
@@ -349,37 +425,38 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
           linear_lr<F>(__shfl(v, lane - 2), __shfl(v, lane - 1), v, __shfl(v, lane + 1),
                        __shfl(v, lane + 2), __shfl(v, lane + 3), qx[0][n], qx[1][n]);
         }
-      } else if constexpr (!DC) {
-#pragma unroll
-        for (int s = 0; s < 6; s++)
-#pragma unroll
-          for (int n = 0; n < 5; n++)
-            qx[s][n] = s == 2 ? q[2][n] : __shfl(q[2][n], lane + s - 2);
       }
       const double jx = xmx * jo, jy = xmy * jo, jz = xmz * jo;
-      const double nxx = 0.5 * (jx + __shfl(jx, lane + 1));
-      const double nxy = 0.5 * (jy + __shfl(jy, lane + 1));
-      const double nxz = 0.5 * (jz + __shfl(jz, lane + 1));
-      if constexpr (DC) {
-        // the float difference to lane+1's node, the differences of lanes
-        // -2..+2 and lane+1's Roe inputs, by shuffles
-        F ex[5], ec[5][5];
-#pragma unroll
-        for (int n = 0; n < 5; n++) ex[n] = (F)(__shfl(q[2][n], lane + 1) - q[2][n]);
+      // (the neighbour's product is rounded: face_normal with j1 = 1)
+      constexpr Rounding rx = rounding<F, HYB>(true);
+      const double nxx = face_normal(rx, xmx, jo, __shfl(jx, lane + 1), 1.0);
+      const double nxy = face_normal(rx, xmy, jo, __shfl(jy, lane + 1), 1.0);
+      const double nxz = face_normal(rx, xmz, jo, __shfl(jz, lane + 1), 1.0);
+      if constexpr (!HYB) {
+        // lane+1's node, the difference to it and those of lanes -2..+2 (and,
+        // in float, lane+1's Roe inputs), by shuffles
+        double qr[5];
+        F ec[5][5];
 #pragma unroll
         for (int n = 0; n < 5; n++) {
-          ec[0][n] = __shfl(ex[n], lane - 2);
-          ec[1][n] = __shfl(ex[n], lane - 1);
-          ec[2][n] = ex[n];
-          ec[3][n] = __shfl(ex[n], lane + 1);
-          ec[4][n] = __shfl(ex[n], lane + 2);
+          qr[n] = __shfl(q[2][n], lane + 1);
+          const F ex = (F)(qr[n] - q[2][n]);
+          ec[0][n] = __shfl(ex, lane - 2);
+          ec[1][n] = __shfl(ex, lane - 1);
+          ec[2][n] = ex;
+          ec[3][n] = __shfl(ex, lane + 1);
+          ec[4][n] = __shfl(ex, lane + 2);
         }
-        const NodeT<F> xr{__shfl(nl.r, lane + 1), __shfl(nl.u, lane + 1), __shfl(nl.v, lane + 1),
-                          __shfl(nl.w, lane + 1), __shfl(nl.H, lane + 1)};
-        F dx[6][5];
-        dev_from_diffs(ec, dx);
-        face_flux_dev<F>(gt, g, dx, q[2], nl, xr, nxx, nxy, nxz, fxr);
-      } else if constexpr (HYB) {
+        if constexpr (DC) {
+          const NodeT<F> xr{__shfl(nl.r, lane + 1), __shfl(nl.u, lane + 1), __shfl(nl.v, lane + 1),
+                            __shfl(nl.w, lane + 1), __shfl(nl.H, lane + 1)};
+          F dx[6][5];
+          dev_from_diffs(ec, dx);
+          face_flux_dev<true>(g, dx, q[2], nl, xr, nxx, nxy, nxz, false, fxr);
+        } else {
+          face_flux(g, ec, q[2], qr, nxx, nxy, nxz, fxr);
+        }
+      } else {
         const int fo = sa.flags_x[o];
         const bool tx = (__shfl(fo, lane - 1) | fo | __shfl(fo, lane + 1)) != 0;
         // qx[0], qx[1]: the reconstructed left and right states
@@ -389,8 +466,6 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
 #pragma unroll
           for (int n = 0; n < 5; n++) fxr[n] = sa.tf_x.flux[n * sa.tf_x.stride + sl];
         }
-      } else {
-        stage_face<F, HYB>(g, qx, nxx, nxy, nxz, false, sa.tf_x, o, fxr);
       }
       if (VIS) {
 #pragma unroll
@@ -401,6 +476,9 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
         }
       }
     }
+    constexpr Rounding rnd = rounding<F, HYB>(false);
+    const double sx = normal(rnd, ax, jo, mx, jb), sy = normal(rnd, ay, jo, my, jb);
+    const double sz = normal(rnd, az, jo, mz, jb);
     if (HYB) {
       t0 = t1;
       t1 = t2;
@@ -409,11 +487,9 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
     if constexpr (DC) {
       F d[6][5];
       dev_from_diffs(e, d);
-      face_flux_dev<F>(gt, g, d, q[2], nl, nr, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz),
-                       f);
+      face_flux_dev<true>(g, d, q[2], nl, nr, sx, sy, sz, AX == 1, f);
     } else {
-      stage_face<F, HYB>(g, q, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz), t0 | t1 | t2,
-                         sa.tf, o, f);
+      stage_face<F, HYB>(g, q, sx, sy, sz, t0 | t1 | t2, sa.tf, o, AX == 1, f);
     }
     if (VIS) {
       const int s0 = vr, s1 = vr == 2 ? 0 : vr + 1, s2 = vr == 0 ? 2 : vr - 1;
@@ -432,20 +508,13 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
       }
       vr = s1;
     }
-    if (!upd) {
-#pragma unroll
-      for (int n = 0; n < 5; n++) fprev[n] = f[n];
-      continue;
-    }
-    double dfx[5];  // xi-face difference (XI)
-    if (XI) {
-#pragma unroll
-      for (int n = 0; n < 5; n++) dfx[n] = fxr[n] - __shfl_up(fxr[n], 1);
-    }
     if (AX == 1) {
 #pragma unroll
       for (int n = 0; n < 5; n++) sa.rhs[n * S + o] = f[n] - fprev[n];
     } else {
+      double dfx[5];  // xi-face difference
+#pragma unroll
+      for (int n = 0; n < 5; n++) dfx[n] = fxr[n] - __shfl_up(fxr[n], 1);
       if (!HOIST) {
 #pragma unroll
         for (int n = 0; n < 5; n++) {
@@ -453,55 +522,10 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
           qnv[n] = sa.stage > 1 ? sa.Qn[n * S + o] : 0.0;
         }
       }
-      const double inv_j = fast_rcp(jo);
-      double qn_out[5];
+      double dg[5];
 #pragma unroll
-      for (int n = 0; n < 5; n++) {
-        double df = rin[n] + (f[n] - fprev[n]);
-        if (XI) df += dfx[n];
-        df *= inv_j;
-        const double qin = q[2][n];
-        double out;
-        if (sa.stage == 1) out = qin - dt * df;
-        else if (sa.stage == 2) out = 0.75 * qnv[n] + 0.25 * (qin - dt * df);
-        else out = (qnv[n] + 2.0 * (qin - dt * df)) * (1.0 / 3.0);
-        qn_out[n] = out;
-      }
-      // primitives of the new state (src/primitive_bc_kernel.cu:63-76)
-      if (own) {
-        double rr, uu, vv, ww, pp;
-        q_to_prim(g, qn_out, rr, uu, vv, ww, pp);
-        const double tt = c.gM2 * pp * fast_rcp(rr);
-        // all stores of a node together, after its arithmetic: with the state's
-        // ahead of the primitives 256^3 took 1610 us for 1531 (hybrid 1203 for
-        // 1165)
-        const auto put = [&](int d) {
-#pragma unroll
-          for (int n = 0; n < 5; n++) sa.Qout[n * S + d] = qn_out[n];
-          if (sa.pmask & 1) sa.prim[d] = rr;
-          if (sa.pmask & 2) sa.prim[S + d] = uu;
-          if (sa.pmask & 4) sa.prim[2 * S + d] = vv;
-          if (sa.pmask & 8) sa.prim[3 * S + d] = ww;
-          if (sa.pmask & 16) sa.prim[4 * S + d] = pp;
-          if (sa.pmask & 32) sa.prim[5 * S + d] = tt;
-        };
-        put(o);
-        if (SHORT && sa.wrap) {
-          // the node's images in the ghosts: along each axis at whose end it
-          // lies, and along each pair and all three of them
-          const int di = i < G ? c.IM : (i >= c.IM - G ? -c.IM : 0);
-          const int dj = t < G ? c.JM : (t >= c.JM - G ? -c.JM : 0);
-          const int dk = m < G ? c.KM : (m >= c.KM - G ? -c.KM : 0);
-          if (di | dj | dk) {
-#pragma unroll 1
-            for (int im = 1; im < 8; im++) {
-              const int ex = im & 1 ? di : 0, ey = im & 2 ? dj : 0, ez = im & 4 ? dk : 0;
-              if ((im & 1 && !ex) || (im & 2 && !ey) || (im & 4 && !ez)) continue;
-              put(o + ex + ey * c.PX + ez * c.PXY);
-            }
-          }
-        }
-      }
+      for (int n = 0; n < 5; n++) dg[n] = f[n] - fprev[n];
+      finish_node<WRAP>(c, sa, g, dt, i, t, m, o, own, dfx, rin, dg, q[2], qnv, jo);
     }
 #pragma unroll
     for (int n = 0; n < 5; n++) fprev[n] = f[n];
@@ -597,10 +621,23 @@ __global__ void __launch_bounds__(256) k_weno_list(Consts c, const int* __restri
   const double* nX = met + (3 * AX + 0) * S;
   const double* nY = met + (3 * AX + 1) * S;
   const double* nZ = met + (3 * AX + 2) * S;
-  const double ax = nX[a] * Ja, ay = nY[a] * Ja, az = nZ[a] * Ja;
-  const double bx = nX[bn] * Jb, by = nY[bn] * Jb, bz = nZ[bn] * Jb;
+  const double nx = face_normal(LEFT, nX[a], Ja, nX[bn], Jb);
+  const double ny = face_normal(LEFT, nY[a], Ja, nY[bn], Jb);
+  const double nz = face_normal(LEFT, nZ[a], Ja, nZ[bn], Jb);
   const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
-  face_flux_form<F>(g, q, 0.5 * (ax + bx), 0.5 * (ay + by), 0.5 * (az + bz), f);
+  if constexpr (sizeof(F) == sizeof(double)) {
+    F e[5][5];
+    stencil_diffs(q, e);
+    face_flux(g, e, q[2], q[3], nx, ny, nz, f);
+  } else {
+    F d[6][5];
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+#pragma unroll
+      for (int m = 0; m < 5; m++) d[s][m] = (F)(q[s][m] - q[2][m]);
+    face_flux_dev<false>(g, d, q[2], node_t<F>(g, q_to_side(g, q[2])),
+                         node_t<F>(g, q_to_side(g, q[3])), nx, ny, nz, false, f);
+  }
 #pragma unroll
   for (int m = 0; m < 5; m++) flux[m * fstride + slot_base + t] = f[m];
 }
@@ -672,11 +709,6 @@ struct MarchCut {
   int parts;   // chunks per CHUNK_MAX nodes
   long waves;  // wavefronts in all
 };
-// Chunks of up to CHUNK_MAX / PARTS_SHORT nodes skip the xi-faces of their first
-// pass by a branch: 64^3 zeta march 41.5 -> 38.5 us.  In long ones the branch
-// parts the arithmetic of the two faces for little: 256^3 1531 us, 1570 with it.
-// From 8 to 16 nodes a chunk both are within the noise.
-constexpr int PARTS_SHORT = 4;
 static MarchCut march_cut(long lines, int n) {
   constexpr long SLOTS = 2048;
   constexpr double PAIR = 1.8;
@@ -699,7 +731,7 @@ static MarchCut march_cut(long lines, int n) {
 }
 
 template <int AX, class F, bool HYB>
-int launch_march(cbns_block* b, StageArgs& sa) {
+int launch_march(cbns_block* b, StageArgs& sa, bool wrap) {
   const Consts& c = b->c;
   const int ax_t = AX == 1 ? 2 : 1;
   const int ni = upd_hi(c, 0) - upd_lo(c, 0) + 1;
@@ -714,8 +746,7 @@ int launch_march(cbns_block* b, StageArgs& sa) {
   const int R = cut.waves <= 1024 ? 1 : MARCH_Y;
   const dim3 grid((unsigned)((nw + R - 1) / R), sa.parts, (nm + CHUNK_MAX - 1) / CHUNK_MAX);
   ProfScope ps(b, AX == 1 ? CBNS_K_MARCH_ETA : CBNS_K_MARCH_ZETA);
-  const bool brief = AX == 2 && (sa.parts >= PARTS_SHORT || sa.wrap);
-  const auto kern = brief ? k_march<AX, F, HYB, AX == 2> : k_march<AX, F, HYB, false>;
+  const auto kern = AX == 2 && wrap ? k_march<AX, F, HYB, AX == 2> : k_march<AX, F, HYB, false>;
   kern<<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
@@ -765,8 +796,8 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
                b->rhs, c.viscous ? b->vtmp : nullptr,
                hyb ? fl + S : nullptr, hyb ? fl : nullptr, pmask,
                TroubledFaces{hyb ? b->tslot + S : nullptr, b->tflux, b->ttotal},
-               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1, stage_wraps(c, dt)};
-  if ((rc = hyb ? launch_march<1, F, true>(b, sa) : launch_march<1, F, false>(b, sa)))
+               TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1};
+  if ((rc = hyb ? launch_march<1, F, true>(b, sa, false) : launch_march<1, F, false>(b, sa, false)))
     return rc;
   if (lam) {
     ProfScope ps(b, CBNS_K_DT);
@@ -777,7 +808,8 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
     sa.flags = fl + 2 * S;
     sa.tf.slot = b->tslot + 2 * S;
   }
-  return hyb ? launch_march<2, F, true>(b, sa) : launch_march<2, F, false>(b, sa);
+  const bool wrap = stage_wraps(c, dt);
+  return hyb ? launch_march<2, F, true>(b, sa, wrap) : launch_march<2, F, false>(b, sa, wrap);
 }
 
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout) {

@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256) k_face_flux(Consts c, Box box, int d,
   const double nx = 0.5 * (met[(3 * d + 0) * S + a] * Ja + met[(3 * d + 0) * S + bb] * Jb);
   const double ny = 0.5 * (met[(3 * d + 1) * S + a] * Ja + met[(3 * d + 1) * S + bb] * Jb);
   const double nz = 0.5 * (met[(3 * d + 2) * S + a] * Ja + met[(3 * d + 2) * S + bb] * Jb);
-  double q[6][5], pl[5], pr[5], f[5];
+  double q[6][5], e[5][5], pl[5], pr[5], f[5];
 #pragma unroll
   for (int s = 0; s < 6; s++)
 #pragma unroll
@@ -41,7 +41,8 @@ __global__ void __launch_bounds__(256) k_face_flux(Consts c, Box box, int d,
   Basis<double> B;
   roe_basis(g, pl[0], pl[1], pl[2], pl[3], pl[4], pr[0], pr[1], pr[2], pr[3], pr[4], nx, ny, nz,
             B);
-  face_flux_basis<double>(g, q, B, nx, ny, nz, f);
+  stencil_diffs(q, e);
+  face_flux_basis(g, e, q[2], q[3], B, nx, ny, nz, f);
 #pragma unroll
   for (int n = 0; n < 5; n++) flux[(d * 5 + n) * S + a] = f[n];
 }

@@ -1,7 +1,7 @@
 // learned.hpp -- device functions of the learned troubled-face indicator.
 //
 //   face_features   30 normalised characteristic stencil differences per face
-//                   (float, on deviations from node m like face_flux_mixed):
+//                   (float, on deviations from node m like face_flux_dev):
 //                   for each characteristic field c of W = L q (L = the
 //                   Roe-averaged left eigenvectors, src/calc_eigenvectors_roe.cu)
 //                   the six stencil values minus the face mean
@@ -70,7 +70,7 @@ __device__ __forceinline__ void char_stencil(const Basis<T>& B, const T d[6][5],
 #pragma unroll
   for (int s = 0; s < 6; s++) {
     const T A = B.K * (d[s][4] - (B.uu * d[s][1] + B.vv * d[s][2] + B.ww * d[s][3]) +
-                       T(0.5) * B.q2 * d[s][0]);
+                       B.k * d[s][0]);
     const T Bn = B.o * (B.qn * d[s][0] - (B.nx * d[s][1] + B.ny * d[s][2] + B.nz * d[s][3]));
     w[0][s] = A + Bn;
     w[1][s] = d[s][0] - T(2) * A;
@@ -140,7 +140,7 @@ __device__ __forceinline__ double face_label(const GasT<double>& g, const double
 
 // Linear-weight face flux.  F = double: the plain arithmetic; F = float: the
 // reconstruction on deviations from node m in float, the states and the flux
-// in double (as face_flux_mixed).
+// in double (as face_flux_dev).
 //   left  = (2 q0 - 13 q1 + 47 q2 + 27 q3 - 3 q4) / 60
 //   right = (2 q5 - 13 q4 + 47 q3 + 27 q2 - 3 q1) / 60
 // one component: the left and right states of the face from its six
@@ -149,13 +149,13 @@ template <class F>
 __device__ __forceinline__ void linear_lr(double v0, double v1, double v2, double v3, double v4,
                                           double v5, double& L, double& R) {
   if constexpr (sizeof(F) == sizeof(double)) {
-    L = (2.0 * v0 - 13.0 * v1 + 47.0 * v2 + 27.0 * v3 - 3.0 * v4) * (1.0 / 60.0);
-    R = (2.0 * v5 - 13.0 * v4 + 47.0 * v3 + 27.0 * v2 - 3.0 * v1) * (1.0 / 60.0);
+    L = fma(-3.0, v4, fma(27.0, v3, fma(47.0, v2, fma(2.0, v0, -(13.0 * v1))))) * (1.0 / 60.0);
+    R = fma(-3.0, v1, fma(27.0, v2, fma(47.0, v3, fma(2.0, v5, -(13.0 * v4))))) * (1.0 / 60.0);
   } else {
     const F d0 = (F)(v0 - v2), d1 = (F)(v1 - v2), d3 = (F)(v3 - v2), d4 = (F)(v4 - v2);
     const F d5 = (F)(v5 - v2);
-    L = v2 + (double)((F(2) * d0 - F(13) * d1 + F(27) * d3 - F(3) * d4) * F(1.0 / 60.0));
-    R = v2 + (double)((F(2) * d5 - F(13) * d4 + F(47) * d3 - F(3) * d1) * F(1.0 / 60.0));
+    L = v2 + (double)(fma(F(-3), d4, fma(F(27), d3, fma(F(2), d0, -(F(13) * d1)))) * F(1.0 / 60.0));
+    R = v2 + (double)(fma(F(-3), d1, fma(F(47), d3, fma(F(2), d5, -(F(13) * d4)))) * F(1.0 / 60.0));
   }
 }
 
@@ -166,7 +166,7 @@ __device__ __forceinline__ void face_linear(const GasT<double>& g, const double 
 #pragma unroll
   for (int c = 0; c < 5; c++)
     linear_lr<F>(q[0][c], q[1][c], q[2][c], q[3][c], q[4][c], q[5][c], qL[c], qR[c]);
-  lf_flux(g, q_to_side(g, qR), q_to_side(g, qL), nx, ny, nz, f);
+  lf_flux<true>(g, q_to_side(g, qR), q_to_side(g, qL), nx, ny, nz, f);
 }
 
 // Logit of this lane's face.  Every lane of the wavefront must call it
