@@ -491,7 +491,7 @@ int cbns_rk3_step(cbns_block* b, double t_end, double* t_cur, double* dt_out) {
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   const double dt = b->h_scalar[2];
   if (std::isnan(dt)) {
-    // the marches left the stages' outputs as they were; so are their ghosts
+    // the stages left their outputs as they were; so are their ghosts
     // filled as a stage would
     if (stage_wraps(b->c, 0.0)) {
       b->step_internal = true;

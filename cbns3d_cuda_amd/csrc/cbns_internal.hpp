@@ -346,17 +346,42 @@ inline int stage_prim_mask(const cbns_block* b, int stage) {
   const int pall = b->c.viscous ? 0x3F : 0x1F;
   return b->step_internal && stage < 3 ? (b->c.viscous ? 0x2E : 0) : pall;
 }
-// The stage's last march writes the ghosts with the state where every axis is
-// periodic, no node reaches the ghosts of both ends and the block is small: a
-// launch less against stores of partial lines that its wavefronts wait for.
-// Step, us, fill launch / march (FP64): inviscid 24^3 93 / 85, 48^3 136 / 136,
-// 96^3 487 / 516; viscous 24^3 121 / 113, 48^3 185 / 182, 64^3 276 / 278, 96^3
-// 710 / 748; the float and hybrid forms cross between 64^3 and 80^3.  (S counts
-// ghosts: 2^18 is 56^3 nodes.)  A time step known to be NaN leaves the state,
-// and its ghosts to the fill.
+// Tiles of x (4 or 16) x 4 x 4 nodes over the updated ones.
+inline long stage_tiles(const Consts& c, int x) {
+  const auto cut = [&](int a, int n) { return (upd_hi(c, a) - upd_lo(c, a) + n) / n; };
+  return (long)cut(0, x) * cut(1, 4) * cut(2, 4);
+}
+// Which way a stage runs: 0 by the marches, 4 or 16 by tiles of that many nodes
+// along xi.  A march of a small block is a chain of faces on a chip mostly idle; a
+// tile4's is one face, and 512 of them run at once (two a CU), so they pay up to
+// two rounds.  tile16 repeats fewer faces (3.6 a node, tile4 3.75) and halo loads;
+// its time goes by the tiles, whose last ones are partly empty, the marches' by the
+// nodes, and from about 10^6 nodes on the marches, which load a node once a sweep,
+// are ahead.  With tiles x (256 tiles / nodes) <= 4096 no block of 17 sizes in three
+// forms, inviscid and viscous, is over 1 % slower than by the marches.  Step, us,
+// by the marches / tile4 / tile16 (FP64 inviscid unless told): 24^3 82 / 44 / 63,
+// 40^3 110 / 72 / 84, 44^3 122 / 89 / 87, 64^3 186 / 190 / 149, viscous 267 / 289 /
+// 225, 128x64x64 303 / 345 / 246, FP32 275 / 341 / 234, 96^3 465 / 526 / 381, viscous
+// FP32 131x75x53 386 / 532 / 376; past the line 104^3 530 / 717 / 512, FP32 469 / 733 /
+// 493, 128^3 883 / 1358 / 892, viscous 1390 / 2243 / 1463; 17x200x200 439 / 519 / 542.
+// (Both limits keep the ghosted block far below 2^29 nodes: at_byte.)
+inline int stage_shape(const Consts& c) {
+  if (stage_tiles(c, 4) <= 1024) return 4;
+  const long t = stage_tiles(c, 16);
+  const long nodes = (long)(upd_hi(c, 0) - upd_lo(c, 0) + 1) * (upd_hi(c, 1) - upd_lo(c, 1) + 1) *
+                     (upd_hi(c, 2) - upd_lo(c, 2) + 1);
+  return t * t <= 16 * nodes ? 16 : 0;
+}
+
+// The tiles write the ghosts with the state where every axis is periodic, no node
+// reaches the ghosts of both ends and the block is small: a launch less against
+// stores of partial lines.  Step, us, fill launch / tiles (FP64 inviscid, FP32
+// viscous): 64^3 147 / 140 and 207 / 198, 80^3 240 / 231 and 333 / 322, 128x64x64 239 /
+// 232 and 332 / 326; beyond (S counts ghosts: 2^20 is 93^3 nodes) no more than the
+// noise.  A time step known to be NaN leaves the state, and its ghosts to the fill.
 inline bool stage_wraps(const Consts& c, double dt) {
   return periodic(c, 0) && periodic(c, 1) && periodic(c, 2) && c.IM >= 2 * G && c.JM >= 2 * G &&
-         c.KM >= 2 * G && c.S <= 1 << 18 && dt == dt;
+         c.KM >= 2 * G && c.S <= 1 << 20 && dt == dt && stage_shape(c) != 0;
 }
 int launch_primitive_all(cbns_block* b, const double* Q);
 int launch_conservative_all(cbns_block* b, double* Q);

@@ -1,4 +1,5 @@
-// k_fused.hip -- one RK3 stage as sweep kernels (cbns_rk3_stage):
+// k_fused.hip -- one RK3 stage (cbns_rk3_stage) as sweep kernels, or on small
+// blocks (stage_shape) as one pass over tiles:
 //
 //   k_march<1>   lanes along i, each thread marches a chunk of nodes along
 //                eta holding the 6-node stencil and the previous face flux in
@@ -15,6 +16,8 @@
 //                the Shu-Osher stage combination, writing the stage output
 //                and its primitives (the boundary pass then only fills
 //                boundaries and ghosts).
+//   k_tile4, k_tile16   the faces along all three axes of a tile of nodes and
+//                its update, in place of both marches
 //
 // Node primitives for the Roe average are recomputed from Q (the
 // primitive array holds exactly f(Q) at every node a face reads:
@@ -112,7 +115,7 @@ template <class F, bool HYB>
 __device__ __forceinline__ void stage_face(const GasT<double>& g, const double q[6][5],
                                            double nx, double ny, double nz, bool troubled,
                                            const TroubledFaces& tf, int face, bool yz,
-                                           double f[5]) {
+                                           double f[5], bool xi = false) {
   if constexpr (!HYB) {
     F e[5][5];
     stencil_diffs(q, e);
@@ -126,7 +129,7 @@ __device__ __forceinline__ void stage_face(const GasT<double>& g, const double q
     }
     return;
   }
-  face_linear<F>(g, q, nx, ny, nz, f);
+  face_linear<F>(g, q, nx, ny, nz, xi, f);
   if (troubled) {
     const long sl = min(max(tf.slot[face], 0), (int)(tf.stride - 1));
 #pragma unroll
@@ -208,8 +211,8 @@ __device__ __forceinline__ void finish_node(const Consts& c, const StageArgs& sa
 }
 
 // AX = 1: march along eta, rhs = dF.  AX = 2: march along zeta with the
-// xi-faces, finish.  WRAP (zeta): also writes the periodic ghosts (stage_wraps).
-template <int AX, class F, bool HYB, bool WRAP>
+// xi-faces, finish.
+template <int AX, class F, bool HYB>
 __global__ void __launch_bounds__(MARCH_X * MARCH_Y)
 __attribute__((amdgpu_waves_per_eu(HYB ? WPE_H : WPE_M, HYB ? WPE_H : WPE_M)))
 k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
@@ -525,11 +528,310 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
       double dg[5];
 #pragma unroll
       for (int n = 0; n < 5; n++) dg[n] = f[n] - fprev[n];
-      finish_node<WRAP>(c, sa, g, dt, i, t, m, o, own, dfx, rin, dg, q[2], qnv, jo);
+      finish_node<false>(c, sa, g, dt, i, t, m, o, own, dfx, rin, dg, q[2], qnv, jo);
     }
 #pragma unroll
     for (int n = 0; n < 5; n++) fprev[n] = f[n];
   }
+}
+
+// A whole stage's fluxes and update in one launch, over tiles of nodes: the
+// workgroup loads the tile's nodes and the three on either side along each axis
+// into LDS, forms every face of the tile, one a lane, into LDS too, and updates
+// the tile's nodes from them.  The faces between tiles are formed twice, but no
+// lane waits for another's faces and dF stays out of memory, so blocks that are
+// small for the marches run this way (stage_shape).  A face's operations are the
+// marches', so the stage has their bits.
+
+// The tile of this workgroup (X x Y x Z nodes from lo on, nx x ny x nz of them in
+// the block); false past the last.  Workgroups go to the 8 XCDs in turn; each XCD
+// takes a run of neighbouring tiles, whose halos its L2 then holds (128^3 viscous
+// step 1739 -> 1566 us, 64^3 259 -> 242).
+constexpr int TILE_XCDS = 8;
+constexpr int TILE_TPB = 256;
+template <int X, int Y, int Z>
+__device__ __forceinline__ bool tile_origin(const int hi[3], int lo[3], int n[3]) {
+  const unsigned tx = (unsigned)(hi[0] - lo[0] + X) / X, ty = (unsigned)(hi[1] - lo[1] + Y) / Y;
+  const unsigned nt = tx * ty * ((unsigned)(hi[2] - lo[2] + Z) / Z);
+  const unsigned t =
+      blockIdx.x % TILE_XCDS * ((nt + TILE_XCDS - 1) / TILE_XCDS) + blockIdx.x / TILE_XCDS;
+  if (t >= nt) return false;
+  const unsigned r = t / tx, q = r / ty;
+  lo[0] += (int)(t - r * tx) * X;
+  lo[1] += (int)(r - q * ty) * Y;
+  lo[2] += (int)q * Z;
+  n[0] = min(X, hi[0] - lo[0] + 1);
+  n[1] = min(Y, hi[1] - lo[1] + 1);
+  n[2] = min(Z, hi[2] - lo[2] + 1);
+  return true;
+}
+
+// Field values by byte offset (below 2^32: stage_shape keeps to small blocks).
+template <class T>
+__device__ __forceinline__ T at_byte(const T* __restrict__ f, unsigned byte) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(f) + byte);
+}
+
+// What a tile's face takes from memory: metrics of its two nodes (o and o + gs,
+// gs the stride of its axis a) and the viscous fluxes around it.
+template <class F>
+struct FaceIn {
+  double j[2], m[3][2];
+  F v[4][4];
+};
+template <class F>
+__device__ __forceinline__ void fetch_face(const Consts& c, const StageArgs& sa,
+                                           const double* __restrict__ met, int a, int gs, int o,
+                                           FaceIn<F>& w) {
+  const long S = c.S;
+  const unsigned o8 = 8u * (unsigned)o, g8 = 8u * (unsigned)gs;
+  const double* __restrict__ nm = met + 3 * a * S;
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    w.j[s] = at_byte(met + JAC * S, o8 + s * g8);
+#pragma unroll
+    for (int d = 0; d < 3; d++) w.m[d][s] = at_byte(nm + d * S, o8 + s * g8);
+  }
+  if (sa.vf) {
+    const int vsh = c.visc_centered ? 0 : -1;
+    const F* __restrict__ v = static_cast<const F*>(sa.vf) + 4 * a * S;
+    const int vo = o + vsh * (1 + c.PX + c.PXY - gs);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+        w.v[e][s] = at_byte(v + e * S, (unsigned)sizeof(F) * (unsigned)(vo + (s - 1) * gs));
+  }
+}
+// Whether a tile's lines along axis a begin where a march's CHUNK_MAX nodes do.
+__device__ __forceinline__ bool first_on_line(const Consts& c, const int lo[3], int a) {
+  return (a == 1 ? lo[1] - upd_lo(c, 1) : lo[2] - upd_lo(c, 2)) % CHUNK_MAX == 0;
+}
+// The face's flux from its stencil q and `w`.  first: the face that opens a
+// march's CHUNK_MAX nodes.
+template <class F, bool HYB>
+__device__ __forceinline__ void tile_face(const Consts& c, const StageArgs& sa,
+                                          const GasT<double>& g, const double q[6][5],
+                                          const FaceIn<F>& w, int a, bool first, int gs, int o,
+                                          double f[5]) {
+  // the products that the marches round
+  const bool left = a == 0 || first;
+  double nv[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+    nv[d] = face_normal(rounding<F, HYB>(left), w.m[d][0], w.j[0], w.m[d][1], w.j[1]);
+  bool troubled = false;
+  TroubledFaces tf = sa.tf_x;
+  if (HYB) {
+    const uint8_t* __restrict__ fl = sa.flags_x + (long)a * c.S;
+    troubled = (fl[o - gs] | fl[o] | fl[o + gs]) != 0;
+    tf.slot += (long)a * c.S;
+  }
+  stage_face<F, HYB>(g, q, nv[0], nv[1], nv[2], troubled, tf, o, a == 1 && !left, f,
+                     a == 0);
+  if (sa.vf) {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      f[e + 1] -= (double)visc_face(w.v[e][0], w.v[e][1], w.v[e][2], w.v[e][3]);
+  }
+}
+
+// Tiles of 4 x 4 x 4 nodes: 240 faces for 256 lanes, a single face long.
+template <class F, bool HYB, bool WRAP>
+__global__ void __launch_bounds__(TILE_TPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_tile4(Consts c, StageArgs sa, const double* __restrict__ met) {
+  constexpr int X = 4, N = X * X * X, L = X * X;  // nodes; lines of an axis
+  // nodes in LDS: the tile's, then each axis' halo, three positions below the
+  // tile and three above, a position of all lines together
+  constexpr int NQ = N + 3 * 6 * L, NF = 3 * (X + 1) * L;
+  __shared__ double sq[5 * NQ], sf[5 * NF];
+  const double dt = sa.dtp ? *sa.dtp : sa.dt;
+  if (!(dt == dt)) return;
+  const long S = c.S;
+  const int tid = threadIdx.x;
+  const int hi[3] = {upd_hi(c, 0), upd_hi(c, 1), upd_hi(c, 2)};
+  int lo[3] = {upd_lo(c, 0), upd_lo(c, 1), upd_lo(c, 2)}, nn[3];
+  if (!tile_origin<X, X, X>(hi, lo, nn)) return;
+#pragma unroll
+  for (int r = 0; r < (NQ + TILE_TPB - 1) / TILE_TPB; r++) {
+    const int t = tid + r * TILE_TPB;
+    int p[3];
+    if (t < N) {
+      p[0] = t % X; p[1] = t / X % X; p[2] = t / L;
+    } else {
+      const int h = t - N, a = h / (6 * L), s = h / L % 6, l = h % L;
+      const int e = s < 3 ? s - 3 : s - 3 + X, u = l % X, v = l / X;
+      p[0] = a == 0 ? e : u;
+      p[1] = a == 1 ? e : (a == 0 ? u : v);
+      p[2] = a == 2 ? e : v;
+    }
+    // nodes past the stencils of the last updated ones are read by no face
+    const int o = idx(c, min(lo[0] + p[0], hi[0] + 3), min(lo[1] + p[1], hi[1] + 3),
+                      min(lo[2] + p[2], hi[2] + 3));
+    if (t < NQ) {
+#pragma unroll
+      for (int n = 0; n < 5; n++) sq[n * NQ + t] = sa.Qin[n * S + o];
+    }
+  }
+  // the lane's face, between positions p - 1 and p of line (u, v) along axis a;
+  // its node o at p - 1
+  const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
+  const int a = tid / ((X + 1) * L), p = tid / L % (X + 1), u = tid % X, v = tid / X % X;
+  const int x = a == 0 ? p - 1 : u, y = a == 1 ? p - 1 : (a == 0 ? u : v), z = a == 2 ? p - 1 : v;
+  const bool has = tid < NF && x < nn[0] && y < nn[1] && z < nn[2];
+  const int o = idx(c, lo[0] + x, lo[1] + y, lo[2] + z);
+  const int gs = a == 0 ? 1 : (a == 1 ? c.PX : c.PXY);
+  FaceIn<F> w;
+  if (has) fetch_face<F>(c, sa, met, a, gs, o, w);
+  __syncthreads();
+  if (has) {
+    const int st = a == 0 ? 1 : (a == 1 ? X : L);
+    const int core = a == 0 ? X * u + L * v : (a == 1 ? u + L * v : u + X * v);
+    const int halo = N + 6 * L * a + tid % L;
+    double q[6][5], f[5];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+      const int pos = p - 3 + s;
+      const int at = pos < 0 ? halo + (pos + 3) * L : (pos >= X ? halo + (pos - X + 3) * L
+                                                                : core + pos * st);
+#pragma unroll
+      for (int n = 0; n < 5; n++) q[s][n] = sq[n * NQ + at];
+    }
+    tile_face<F, HYB>(c, sa, g, q, w, a, p == 0 && first_on_line(c, lo, a), gs, o, f);
+#pragma unroll
+    for (int n = 0; n < 5; n++) sf[n * NF + tid] = f[n];
+  }
+  __syncthreads();
+  if (tid < N) {
+    const int x = tid % X, y = tid / X % X, z = tid / L;
+    if (x >= nn[0] || y >= nn[1] || z >= nn[2]) return;
+    const int i = lo[0] + x, j = lo[1] + y, k = lo[2] + z, o = idx(c, i, j, k);
+    // face p of line (u, v) of axis a at (5 a + p) L + u + X v
+    const int fe = x * L + y + X * z, ff = (5 + y) * L + x + X * z, fg = (10 + z) * L + x + X * y;
+    double de[5], df[5], dg[5], qin[5], qn[5];
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+      qn[n] = sa.stage > 1 ? sa.Qn[n * S + o] : 0.0;
+      qin[n] = sq[n * NQ + tid];
+      const double* s = sf + n * NF;
+      de[n] = s[fe + L] - s[fe];
+      df[n] = s[ff + L] - s[ff];
+      dg[n] = s[fg + L] - s[fg];
+    }
+    finish_node<WRAP>(c, sa, g, dt, i, j, k, o, true, de, df, dg, qin, qn, met[JAC * S + o]);
+  }
+}
+
+// Tiles of 16 x 4 x 4 nodes, a node a lane for the update.  Their faces are
+// handed to the wavefronts by position: the 64 of one position along eta or zeta,
+// 4 lines of 16 along xi, and the 17th of the 16 lines, so the axis, and along
+// eta and zeta the position too, are the wavefront's and cost the lanes no
+// arithmetic.
+template <class F, bool HYB, bool WRAP>
+__global__ void __launch_bounds__(TILE_TPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_tile16(Consts c, StageArgs sa, const double* __restrict__ met) {
+  constexpr int X = 16, Y = 4, R = X + 6;  // a row's nodes in LDS, xi-halo included
+  // nodes in LDS: the rows (y + 4 z), then 3 + 3 positions along eta, then along
+  // zeta, 64 nodes each
+  constexpr int HY = R * Y * Y, HZ = HY + 6 * 64, NQ = HZ + 6 * 64;
+  constexpr int FZ = (Y + 1) * 64, FX = 2 * FZ, NF = FX + (X + 1) * Y * Y;
+  constexpr int CHUNKS = 15;
+  __shared__ double sq[5 * NQ], sf[5 * NF];
+  const double dt = sa.dtp ? *sa.dtp : sa.dt;
+  if (!(dt == dt)) return;
+  const long S = c.S;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hi[3] = {upd_hi(c, 0), upd_hi(c, 1), upd_hi(c, 2)};
+  int lo[3] = {upd_lo(c, 0), upd_lo(c, 1), upd_lo(c, 2)}, nn[3];
+  if (!tile_origin<X, Y, Y>(hi, lo, nn)) return;
+  // nodes past the stencils of the last updated ones are read by no face
+  const auto node = [&](int x, int y, int z) {
+    return idx(c, min(lo[0] + x, hi[0] + 3), min(lo[1] + y, hi[1] + 3), min(lo[2] + z, hi[2] + 3));
+  };
+  const int lx = lane % X, lv = lane / X;
+  {
+    double h[5][5];
+    int to[5];
+#pragma unroll
+    for (int r = 0; r < 5; r++) {
+      int x, y, z;
+      if (r < 2) {
+        const int t = tid + r * TILE_TPB;
+        x = t % R - 3; y = t / R % Y; z = t / (R * Y);
+        to[r] = t;
+      } else {
+        const int p = 4 * (r - 2) + wv, s = p % 6, e = s < 3 ? s - 3 : s - 3 + Y;
+        x = lx;
+        y = p < 6 ? e : lv;
+        z = p < 6 ? lv : e;
+        to[r] = HY + 64 * p + lane;
+      }
+      const unsigned o8 = 8u * (unsigned)node(x, y, z);
+#pragma unroll
+      for (int n = 0; n < 5; n++) h[r][n] = at_byte(sa.Qin + n * S, o8);
+    }
+#pragma unroll
+    for (int r = 0; r < 5; r++)
+#pragma unroll
+      for (int n = 0; n < 5; n++)
+        if (r != 1 || to[r] < HY) sq[n * NQ + to[r]] = h[r][n];
+  }
+  const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
+  __syncthreads();
+#pragma unroll 1
+  for (int ch = wv; ch < CHUNKS; ch += TILE_TPB / 64) {
+    // chunk 0-4: eta, position ch; 5-9: zeta, position ch - 5; 10-13: xi, lines of
+    // plane ch - 10, positions 0-15; 14: xi, position 16
+    const int a = ch < 5 ? 1 : (ch < 10 ? 2 : 0);
+    const int p = a == 1 ? ch : ch - 5;  // eta and zeta: the faces' position
+    int x = lx, y = lv, z = lv;
+    if (a == 1) y = p - 1;
+    else if (a == 2) z = p - 1;
+    else if (ch < 14) { x = lx - 1; z = ch - 10; }
+    else { x = X - 1; y = lane % Y; z = lane / Y; }
+    if (x >= nn[0] || y >= nn[1] || z >= nn[2]) continue;
+    const int gs = a == 0 ? 1 : (a == 1 ? c.PX : c.PXY);
+    const int o = idx(c, lo[0] + x, lo[1] + y, lo[2] + z);
+    FaceIn<F> w;
+    fetch_face<F>(c, sa, met, a, gs, o, w);
+    // position s of the stencil: in the rows at row + s (xi) or row + pos * st, or
+    // in the halo of the axis
+    const int row = a == 1 ? lx + 3 + R * Y * lv
+                           : (a == 2 ? lx + 3 + R * lv : x + 1 + R * (y + Y * z));
+    const int halo = (a == 1 ? HY : HZ) + lane, st = a == 1 ? R : R * Y;
+    double q[6][5], f[5];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+      const int pos = p - 3 + s;
+      const int at = a == 0 ? row + s
+                            : ((unsigned)pos < (unsigned)Y
+                                   ? row + pos * st
+                                   : halo + 64 * (pos < 0 ? pos + 3 : pos - Y + 3));
+#pragma unroll
+      for (int n = 0; n < 5; n++) q[s][n] = sq[n * NQ + at];
+    }
+    tile_face<F, HYB>(c, sa, g, q, w, a, p == 0 && first_on_line(c, lo, a), gs, o, f);
+    const int to = a == 0 ? FX + (X + 1) * (y + Y * z) + x + 1 : 64 * ch + lane;
+#pragma unroll
+    for (int n = 0; n < 5; n++) sf[n * NF + to] = f[n];
+  }
+  __syncthreads();
+  const int x = lx, y = lv, z = wv;
+  if (x >= nn[0] || y >= nn[1] || z >= nn[2]) return;
+  const int i = lo[0] + x, j = lo[1] + y, k = lo[2] + z, o = idx(c, i, j, k);
+  const int fe = FX + (X + 1) * (y + Y * z) + x, ff = 64 * y + x + X * z, fg = FZ + 64 * z + x + X * y;
+  double de[5], df[5], dg[5], qin[5], qn[5];
+#pragma unroll
+  for (int n = 0; n < 5; n++) {
+    qn[n] = sa.stage > 1 ? sa.Qn[n * S + o] : 0.0;
+    qin[n] = sq[n * NQ + x + 3 + R * (y + Y * z)];
+    const double* s = sf + n * NF;
+    de[n] = s[fe + 1] - s[fe];
+    df[n] = s[ff + 64] - s[ff];
+    dg[n] = s[fg + 64] - s[fg];
+  }
+  finish_node<WRAP>(c, sa, g, dt, i, j, k, o, true, de, df, dg, qin, qn, met[JAC * S + o]);
 }
 
 // The troubled faces of axis AX in the flux kernels' face range fb: face m
@@ -731,7 +1033,7 @@ static MarchCut march_cut(long lines, int n) {
 }
 
 template <int AX, class F, bool HYB>
-int launch_march(cbns_block* b, StageArgs& sa, bool wrap) {
+int launch_march(cbns_block* b, StageArgs& sa) {
   const Consts& c = b->c;
   const int ax_t = AX == 1 ? 2 : 1;
   const int ni = upd_hi(c, 0) - upd_lo(c, 0) + 1;
@@ -746,8 +1048,18 @@ int launch_march(cbns_block* b, StageArgs& sa, bool wrap) {
   const int R = cut.waves <= 1024 ? 1 : MARCH_Y;
   const dim3 grid((unsigned)((nw + R - 1) / R), sa.parts, (nm + CHUNK_MAX - 1) / CHUNK_MAX);
   ProfScope ps(b, AX == 1 ? CBNS_K_MARCH_ETA : CBNS_K_MARCH_ZETA);
-  const auto kern = AX == 2 && wrap ? k_march<AX, F, HYB, AX == 2> : k_march<AX, F, HYB, false>;
-  kern<<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
+  k_march<AX, F, HYB><<<grid, dim3(MARCH_X, R), 0, b->stream>>>(c, sa, b->met);
+  CBNS_HIP(b, hipGetLastError());
+  return CBNS_OK;
+}
+
+template <class F, bool HYB>
+int launch_tiles(cbns_block* b, const StageArgs& sa, int x, bool wrap) {
+  const unsigned grid = (unsigned)((stage_tiles(b->c, x) + TILE_XCDS - 1) / TILE_XCDS * TILE_XCDS);
+  ProfScope ps(b, CBNS_K_MARCH_ZETA);
+  const auto kern = x == 4 ? (wrap ? k_tile4<F, HYB, true> : k_tile4<F, HYB, false>)
+                           : (wrap ? k_tile16<F, HYB, true> : k_tile16<F, HYB, false>);
+  kern<<<grid, TILE_TPB, 0, b->stream>>>(b->c, sa, b->met);
   CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
 }
@@ -761,7 +1073,7 @@ int viscous_part(cbns_block* b, double* lam, int parts) {
 constexpr int TFULL_EVERY = 8;  // steps between indicator passes while a list overflows
 
 // One fused stage: [indicator and face lists (hybrid, when due)], viscous
-// flux pass, eta march, zeta march.  The flux pass reads only the stage
+// flux pass, then the tiles or the eta march and the zeta march.  The flux pass reads only the stage
 // input's primitives, so it may run before the eta march; the marches
 // difference its node fluxes along with the inviscid face fluxes.
 template <class F>
@@ -797,19 +1109,22 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
                hyb ? fl + S : nullptr, hyb ? fl : nullptr, pmask,
                TroubledFaces{hyb ? b->tslot + S : nullptr, b->tflux, b->ttotal},
                TroubledFaces{hyb ? b->tslot : nullptr, b->tflux, b->ttotal}, 1};
-  if ((rc = hyb ? launch_march<1, F, true>(b, sa, false) : launch_march<1, F, false>(b, sa, false)))
+  const int shape = stage_shape(c);
+  if (!shape && (rc = hyb ? launch_march<1, F, true>(b, sa) : launch_march<1, F, false>(b, sa)))
     return rc;
   if (lam) {
     ProfScope ps(b, CBNS_K_DT);
     if ((rc = launch_dt_from_partials(b, lam, (int)visc_flux_blocks(c), b->dt_cap, b->red + 2)))
       return rc;
   }
+  if (shape)
+    return hyb ? launch_tiles<F, true>(b, sa, shape, stage_wraps(c, dt))
+               : launch_tiles<F, false>(b, sa, shape, stage_wraps(c, dt));
   if (hyb) {
     sa.flags = fl + 2 * S;
     sa.tf.slot = b->tslot + 2 * S;
   }
-  const bool wrap = stage_wraps(c, dt);
-  return hyb ? launch_march<2, F, true>(b, sa, wrap) : launch_march<2, F, false>(b, sa, wrap);
+  return hyb ? launch_march<2, F, true>(b, sa) : launch_march<2, F, false>(b, sa);
 }
 
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout) {

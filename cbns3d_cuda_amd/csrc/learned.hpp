@@ -159,14 +159,16 @@ __device__ __forceinline__ void linear_lr(double v0, double v1, double v2, doubl
   }
 }
 
+// xi: a xi-face (lf_flux's SWAP is the others').
 template <class F>
 __device__ __forceinline__ void face_linear(const GasT<double>& g, const double q[6][5], double nx,
-                                            double ny, double nz, double f[5]) {
+                                            double ny, double nz, bool xi, double f[5]) {
   double qL[5], qR[5];
 #pragma unroll
   for (int c = 0; c < 5; c++)
     linear_lr<F>(q[0][c], q[1][c], q[2][c], q[3][c], q[4][c], q[5][c], qL[c], qR[c]);
-  lf_flux<true>(g, q_to_side(g, qR), q_to_side(g, qL), nx, ny, nz, f);
+  if (xi) lf_flux<false>(g, q_to_side(g, qR), q_to_side(g, qL), nx, ny, nz, f);
+  else lf_flux<true>(g, q_to_side(g, qR), q_to_side(g, qL), nx, ny, nz, f);
 }
 
 // Logit of this lane's face.  Every lane of the wavefront must call it
