@@ -478,7 +478,7 @@ int cbns_rk3_step(cbns_block* b, double t_end, double* t_cur, double* dt_out) {
   b->dt_cap = t_end - *t_cur;
   if (!b->c.viscous) {
     ProfScope ps(b, CBNS_K_DT);
-    if ((rc = launch_dt_device(b, b->dt_cap, b->red + 2))) return rc;
+    if ((rc = launch_dt_device(b, b->dt_cap, b->red + 2, b->h_scalar + 2))) return rc;
   }
   b->dt_fold = true;
   b->step_internal = true;
@@ -486,8 +486,6 @@ int cbns_rk3_step(cbns_block* b, double t_end, double* t_cur, double* dt_out) {
   b->dt_fold = false;
   b->step_internal = false;
   if (rc) return rc;
-  CBNS_HIP(b, hipMemcpyAsync(b->h_scalar + 2, b->red + 2, 2 * sizeof(double),
-                             hipMemcpyDeviceToHost, b->stream));
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   const double dt = b->h_scalar[2];
   if (std::isnan(dt)) {

@@ -394,14 +394,15 @@ int launch_viscous(cbns_block* b, double* vf, double* out, int mode, double* lam
 int launch_viscous_f32(cbns_block* b, double* scratch, double* rhs, double* lam_part = nullptr,
                        int parts = 3);
 long visc_flux_blocks(const Consts& c);
-int launch_dt_from_partials(cbns_block* b, const double* partial, int n, double cap,
-                            double* out);
+int launch_dt_from_partials(cbns_block* b, const double* partial, int n, double cap, double* out,
+                            double* host);
 int launch_update_rk3(cbns_block* b, double dt, int stage);
 int launch_calc_dt(cbns_block* b, double* dt_host);
 // workgroups (partial maxima) of the time-step pass, and the pass itself
-// with dt (limited to cap) and the maximum left in out[0..1] on the device
+// with dt (limited to cap) and the maximum left in out[0..1] on the device and
+// in host[0..1] (pinned memory, valid once the stream is done)
 long time_step_blocks(const Consts& c);
-int launch_dt_device(cbns_block* b, double cap, double* out);
+int launch_dt_device(cbns_block* b, double cap, double* out, double* host);
 int launch_sutherland(cbns_block* b);
 int launch_fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* qout);
 int launch_fill(hipStream_t s, double* p, long n, double v);

@@ -1114,7 +1114,7 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
     return rc;
   if (lam) {
     ProfScope ps(b, CBNS_K_DT);
-    if ((rc = launch_dt_from_partials(b, lam, (int)visc_flux_blocks(c), b->dt_cap, b->red + 2)))
+    if ((rc = launch_dt_from_partials(b, lam, (int)visc_flux_blocks(c), b->dt_cap, b->red + 2, b->h_scalar + 2)))
       return rc;
   }
   if (shape)
