@@ -903,26 +903,35 @@ __global__ void __launch_bounds__(256) k_face_list(Consts c, Box fb,
   }
 }
 
-// Characteristic-WENO flux (the stage's arithmetic form) of each listed face
-// of axis AX, from the stage input Q, into its slot.
-template <int AX, class F>
-__global__ void __launch_bounds__(256) k_weno_list(Consts c, const int* __restrict__ list,
-                                                   unsigned n, const double* __restrict__ Q,
+// Characteristic-WENO flux (the stage's arithmetic form) of each listed face, from
+// the stage input Q, into its slot: the lists of the three axes in one launch, n[a]
+// faces of axis a from slot off[a] on, over workgroups from first[a] on (three
+// launches left the chip idle between them: 92 -> 78 us on the 256x128x128
+// shock-vortex block, 24 -> 16 on the 256^3 vortex; what is left is the gather of the
+// stencils).
+struct WenoLists {
+  unsigned n[3], first[3];
+  int off[3];
+};
+template <class F>
+__global__ void __launch_bounds__(256) k_weno_list(Consts c, WenoLists wl,
+                                                   const int* __restrict__ list,
+                                                   const double* __restrict__ Q,
                                                    const double* __restrict__ met,
-                                                   double* __restrict__ flux, long fstride,
-                                                   int slot_base) {
-  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const long S = c.S;
-  const int st = stride(c, AX);
-  const int a = list[t], bn = a + st;
+                                                   double* __restrict__ flux, long fstride) {
+  const int ax = blockIdx.x >= wl.first[2] ? 2 : (blockIdx.x >= wl.first[1] ? 1 : 0);
+  const unsigned t = (blockIdx.x - wl.first[ax]) * blockDim.x + threadIdx.x;
+  if (t >= wl.n[ax]) return;
+  const long S = c.S, slot = wl.off[ax] + (long)t;
+  const int st = stride(c, ax);
+  const int a = list[slot], bn = a + st;
   double q[6][5], f[5];
 #pragma unroll
   for (int s = 0; s < 6; s++) load_q(Q, S, a + (s - 2) * st, q[s]);
   const double Ja = met[JAC * S + a], Jb = met[JAC * S + bn];
-  const double* nX = met + (3 * AX + 0) * S;
-  const double* nY = met + (3 * AX + 1) * S;
-  const double* nZ = met + (3 * AX + 2) * S;
+  const double* nX = met + (3 * ax + 0) * S;
+  const double* nY = met + (3 * ax + 1) * S;
+  const double* nZ = met + (3 * ax + 2) * S;
   const double nx = face_normal(LEFT, nX[a], Ja, nX[bn], Jb);
   const double ny = face_normal(LEFT, nY[a], Ja, nY[bn], Jb);
   const double nz = face_normal(LEFT, nZ[a], Ja, nZ[bn], Jb);
@@ -941,7 +950,7 @@ __global__ void __launch_bounds__(256) k_weno_list(Consts c, const int* __restri
                          node_t<F>(g, q_to_side(g, q[3])), nx, ny, nz, false, f);
   }
 #pragma unroll
-  for (int m = 0; m < 5; m++) flux[m * fstride + slot_base + t] = f[m];
+  for (int m = 0; m < 5; m++) flux[m * fstride + slot] = f[m];
 }
 
 template <int AX>
@@ -955,17 +964,18 @@ void launch_face_list_axis(cbns_block* b, const Box& fb) {
 template <class F>
 int launch_weno_lists(cbns_block* b, const double* qin) {
   ProfScope ps(b, CBNS_K_WENO_LIST);
+  WenoLists wl;
+  unsigned groups = 0;
   for (int a = 0; a < 3; a++) {
-    const unsigned n = b->h_tcount[a];
-    if (n == 0) continue;
-    const unsigned nb = (n + 255) / 256;
-    const int sb = (int)b->toff[a];
-    const int* lst = b->tlist + b->toff[a];
-    if (a == 0) k_weno_list<0, F><<<nb, 256, 0, b->stream>>>(b->c, lst, n, qin, b->met, b->tflux, b->ttotal, sb);
-    else if (a == 1) k_weno_list<1, F><<<nb, 256, 0, b->stream>>>(b->c, lst, n, qin, b->met, b->tflux, b->ttotal, sb);
-    else k_weno_list<2, F><<<nb, 256, 0, b->stream>>>(b->c, lst, n, qin, b->met, b->tflux, b->ttotal, sb);
-    CBNS_HIP(b, hipGetLastError());
+    wl.n[a] = b->h_tcount[a];
+    wl.first[a] = groups;
+    wl.off[a] = (int)b->toff[a];
+    groups += (wl.n[a] + 255) / 256;
   }
+  if (groups == 0) return CBNS_OK;
+  k_weno_list<F><<<groups, 256, 0, b->stream>>>(b->c, wl, b->tlist, qin, b->met, b->tflux,
+                                                b->ttotal);
+  CBNS_HIP(b, hipGetLastError());
   return CBNS_OK;
 }
 
