@@ -340,11 +340,16 @@ int launch_bc_primitive(cbns_block* b, double* Q);
 int launch_bc_only(cbns_block* b, double* Q, int pmask = -1);
 // Primitives a fused stage's output needs: all of them, except inside
 // cbns_rk3_step, where the first two stages' outputs feed only the next
-// stage (the marches derive what they need from Q; the viscous flux pass
-// reads u, v, w, T) and the third stage writes all of them.
+// stage (the marches derive what they need from Q; so does the viscous flux pass
+// where every axis is periodic, elsewhere it reads u, v, w, T, which boundary rules
+// set) and the third stage writes all of them.
+inline bool flux_pass_from_q(const Consts& c) {
+  return c.viscous && periodic(c, 0) && periodic(c, 1) && periodic(c, 2);
+}
 inline int stage_prim_mask(const cbns_block* b, int stage) {
   const int pall = b->c.viscous ? 0x3F : 0x1F;
-  return b->step_internal && stage < 3 ? (b->c.viscous ? 0x2E : 0) : pall;
+  if (!b->step_internal || stage == 3) return pall;
+  return b->c.viscous && !flux_pass_from_q(b->c) ? 0x2E : 0;
 }
 // Tiles of x (4 or 16) x 4 x 4 nodes over the updated ones.
 inline long stage_tiles(const Consts& c, int x) {
@@ -389,10 +394,12 @@ int launch_freestream(cbns_block* b);
 int launch_numerical_flux(cbns_block* b, const double* Q);
 int launch_viscous_unfused(cbns_block* b);
 // parts: 1 the flux pass, 2 the divergence pass, 3 both
+// q: the flux pass forms its primitives from this state (periodic blocks, no
+// lam_part)
 int launch_viscous(cbns_block* b, double* vf, double* out, int mode, double* lam_part = nullptr,
-                   int parts = 3);
+                   int parts = 3, const double* q = nullptr);
 int launch_viscous_f32(cbns_block* b, double* scratch, double* rhs, double* lam_part = nullptr,
-                       int parts = 3);
+                       int parts = 3, const double* q = nullptr);
 long visc_flux_blocks(const Consts& c);
 int launch_dt_from_partials(cbns_block* b, const double* partial, int n, double cap, double* out,
                             double* host);

@@ -1075,9 +1075,9 @@ int launch_tiles(cbns_block* b, const StageArgs& sa, int x, bool wrap) {
 }
 
 template <class F>
-int viscous_part(cbns_block* b, double* lam, int parts) {
-  return sizeof(F) == sizeof(double) ? launch_viscous(b, b->vtmp, b->rhs, 1, lam, parts)
-                                     : launch_viscous_f32(b, b->vtmp, b->rhs, lam, parts);
+int viscous_fluxes(cbns_block* b, double* lam, const double* q) {
+  return sizeof(F) == sizeof(double) ? launch_viscous(b, b->vtmp, b->rhs, 1, lam, 1, q)
+                                     : launch_viscous_f32(b, b->vtmp, b->rhs, lam, 1, q);
 }
 
 constexpr int TFULL_EVERY = 8;  // steps between indicator passes while a list overflows
@@ -1107,7 +1107,9 @@ int fused_stage(cbns_block* b, double dt, int stage, const double* qin, double* 
   }
   // first stage of a folded step: the flux pass also forms dt
   double* lam = c.viscous && b->dt_fold && stage == 1 ? b->lam_part : nullptr;
-  if (c.viscous && (rc = viscous_part<F>(b, lam, 1))) return rc;
+  // inside a step the first two stages leave periodic blocks no primitives
+  const bool from_q = b->step_internal && stage > 1 && flux_pass_from_q(c);
+  if (c.viscous && (rc = viscous_fluxes<F>(b, lam, from_q ? qin : nullptr))) return rc;
   // more troubled faces than the lists hold: WENO at every face
   const bool hyb = hyb_form && !b->tfull;
   if (hyb && (rc = launch_weno_lists<F>(b, qin))) return rc;

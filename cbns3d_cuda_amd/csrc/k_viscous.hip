@@ -40,6 +40,7 @@
 // its six waves per SIMD and 20 % of its time, and a plane buffer for Fv saved
 // nothing (it is bound by its HBM bytes).
 #include "cbns_internal.hpp"
+#include "face_math.hpp"
 
 namespace cbns {
 
@@ -70,12 +71,6 @@ constexpr int FROWS = VISC_FLUX_ROWS;
 // 4th-order central difference from the values at -2, -1, +1, +2
 __device__ __forceinline__ double central4(double a, double b, double d, double e) {
   return fma(-1.0 / 12.0, e, fma(2.0 / 3.0, d, fma(1.0 / 12.0, a, -(2.0 / 3.0 * b))));
-}
-
-// a0 b0 + a1 b1 + a2 b2
-template <class T>
-__device__ __forceinline__ T dot3(T a0, T b0, T a1, T b1, T a2, T b2) {
-  return fma(a2, b2, fma(a0, b0, a1 * b1));
 }
 
 // 4th-order derivatives of the four fields f at node offset o on one of the two
@@ -142,12 +137,13 @@ template <class T>
 __device__ __forceinline__ double visc_node_fluxes(const Consts& c, const double du[4][3],
                                                    const double uvw[3], double T_l,
                                                    const double m[10], T E[3][4]) {
+#pragma clang fp contract(off)
   T g[4][3];
 #pragma unroll
   for (int a = 0; a < 4; a++) {
     const T d0 = (T)du[a][0], d1 = (T)du[a][1], d2 = (T)du[a][2];
 #pragma unroll
-    for (int b = 0; b < 3; b++) g[a][b] = dot3(d0, (T)m[b], d1, (T)m[3 + b], d2, (T)m[6 + b]);
+    for (int b = 0; b < 3; b++) g[a][b] = sum3(d0, (T)m[b], d1, (T)m[3 + b], d2, (T)m[6 + b]);
   }
   const double mu_d = (1.0 + c.C_T_inf) / (T_l + c.C_T_inf) * sqrt(T_l * T_l * T_l);
   const T mr = (T)(mu_d * c.Re_inv);
@@ -163,14 +159,14 @@ __device__ __forceinline__ double visc_node_fluxes(const Consts& c, const double
   T e[3];  // u . tau - q
 #pragma unroll
   for (int b = 0; b < 3; b++)
-    e[b] = fma(-mq, g[3][b], dot3((T)uvw[0], tau[0][b], (T)uvw[1], tau[1][b], (T)uvw[2], tau[2][b]));
+    e[b] = fma(-mq, g[3][b], sum3((T)uvw[0], tau[0][b], (T)uvw[1], tau[1][b], (T)uvw[2], tau[2][b]));
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const T nx = (T)(m[3 * d + 0] * m[JAC]), ny = (T)(m[3 * d + 1] * m[JAC]);
     const T nz = (T)(m[3 * d + 2] * m[JAC]);
 #pragma unroll
-    for (int a = 0; a < 3; a++) E[d][a] = dot3(nx, tau[0][a], ny, tau[1][a], nz, tau[2][a]);
-    E[d][3] = dot3(nx, e[0], ny, e[1], nz, e[2]);
+    for (int a = 0; a < 3; a++) E[d][a] = sum3(nx, tau[0][a], ny, tau[1][a], nz, tau[2][a]);
+    E[d][3] = sum3(nx, e[0], ny, e[1], nz, e[2]);
   }
   return mu_d;
 }
@@ -211,9 +207,16 @@ __device__ inline bool visc_flux_lane(const TileMarch& t, int& i, int& j, int& k
 // written to lam_part[workgroup]; NaN if any node's is NaN.
 // REF: the block has a reference axis (one-sided derivatives at its two outer
 // layers); a periodic block's kernel holds no branch on the position.
-template <class T, bool LAM, bool REF>
+// FROMQ: u, v, w, T are formed from the conservative state Q, bit for bit as the
+// stage that wrote it would have, and no primitives are read: the pass has one field
+// more to load (128^3 134 -> 141 us, 256^3 1026 -> 1042), the stage before it four
+// fewer to store and to wrap (256^3 precision form: zeta march 1143 -> 1042, ghosts 68 ->
+// 51; FP64 1459 -> 1446).  Steps: 128^3 1375 -> 1336 us, 256^3 9580 -> 9500, hybrid 9370
+// -> 9040.
+template <class T, bool LAM, bool REF, bool FROMQ>
 __global__ void __launch_bounds__(64 * FROWS) k_visc_fluxes(Consts c, TileMarch tm,
                                                      const double* __restrict__ prim,
+                                                     const double* __restrict__ Q,
                                                      const double* __restrict__ met,
                                                      T* __restrict__ vf,
                                                      double* __restrict__ lam_part) {
@@ -232,30 +235,53 @@ __global__ void __launch_bounds__(64 * FROWS) k_visc_fluxes(Consts c, TileMarch 
   const long S = c.S;
   const int sz = c.PXY;
   const double* f0[4] = {prim + P_U * S, prim + P_V * S, prim + P_W * S, prim + P_T * S};
+  // what is loaded of a node, and its u, v, w, T
+  constexpr int NL = FROMQ ? 5 : 4;
+  const auto fetch = [&](int o, double v[NL]) {
+#pragma unroll
+    for (int f = 0; f < NL; f++) v[f] = FROMQ ? Q[f * S + o] : f0[f][o];
+  };
+  const auto uvwt = [&](const double v[NL], double w[4]) {
+    if constexpr (FROMQ) {
+      const GasT<double> g{c.gamma, c.gam1, c.gam1_inv};
+      double r, p;
+      q_to_prim(g, v, r, w[0], w[1], w[2], p);
+      w[3] = c.gM2 * p * fast_rcp(r);
+    } else {
+#pragma unroll
+      for (int f = 0; f < 4; f++) w[f] = v[f];
+    }
+  };
   // lanes and rows past the array load its last ones (their values feed no
   // node of the box)
   const int ic = min(i, c.IM + G - 1);
   const int base = idx(c, ic, min(j, c.JM + G - 1), 0);
   const int hbase = idx(c, ic, min(jh, c.JM + G - 1), 0);
-  double win[4][5], hn[4];
+  double win[4][5], hn[NL];
+  {
+    double v[4][NL];
 #pragma unroll
-  for (int f = 0; f < 4; f++) {
+    for (int s = 0; s < 4; s++) fetch(base + (k0 - 2 + s) * sz, v[s]);
+    fetch(hbase + k0 * sz, hn);
 #pragma unroll
-    for (int s = 0; s < 4; s++) win[f][s + 1] = f0[f][base + (k0 - 2 + s) * sz];
-    hn[f] = f0[f][hbase + k0 * sz];
+    for (int s = 0; s < 4; s++) {
+      double w[4];
+      uvwt(v[s], w);
+#pragma unroll
+      for (int f = 0; f < 4; f++) win[f][s + 1] = w[f];
+    }
   }
   for (int k = k0; k < k1; k++) {
     // every load of the plane up front (the halo rows of the next plane, which
     // the barrier would wait for)
-    double hv[4], m[10], rp[2] = {1.0, 1.0};
+    double hv[4], m[10], rp[2] = {1.0, 1.0}, pn[NL];
 #pragma unroll
-    for (int f = 0; f < 4; f++) {
+    for (int f = 0; f < 4; f++)
 #pragma unroll
       for (int s = 0; s < 4; s++) win[f][s] = win[f][s + 1];
-      win[f][4] = f0[f][base + (k + 2) * sz];
-      hv[f] = hn[f];
-      hn[f] = f0[f][hbase + (k + 1) * sz];
-    }
+    uvwt(hn, hv);
+    fetch(base + (k + 2) * sz, pn);
+    fetch(hbase + (k + 1) * sz, hn);
 #pragma unroll
     for (int q = 0; q < 10; q++) m[q] = met[q * S + base + k * sz];
     if (LAM) {
@@ -277,6 +303,12 @@ __global__ void __launch_bounds__(64 * FROWS) k_visc_fluxes(Consts c, TileMarch 
     // keeps the metric loads ahead of the barrier (they would sink to their use)
 #pragma unroll
     for (int q = 0; q < 10; q++) asm volatile("" : "+v"(m[q]));
+    {
+      double w[4];
+      uvwt(pn, w);
+#pragma unroll
+      for (int f = 0; f < 4; f++) win[f][4] = w[f];
+    }
 #pragma unroll
     for (int f = 0; f < 4; f++) {
       du[f][1] = central4(plane[pb][f][ty][lane], plane[pb][f][ty + 1][lane],
@@ -398,17 +430,23 @@ long visc_flux_blocks(const Consts& c) { return (long)tile_march_blocks(visc_flu
 // `out`, mode 1 subtracts the divergence from the right-hand side (5*S).
 // lam_part (visc_flux_blocks entries) or null: the flux pass also forms the
 // time step's per-workgroup spectral-radius maxima.
+// q: the state to take u, v, w, T from, or null (the primitives).
 template <class T>
-int viscous(cbns_block* b, T* vf, double* out, int mode, double* lam_part, int parts) {
+int viscous(cbns_block* b, T* vf, double* out, int mode, double* lam_part, int parts,
+            const double* q) {
   const Consts& c = b->c;
   if (parts & 1) {
     ProfScope ps(b, CBNS_K_VISC_FLUX);
     const TileMarch tm = visc_flux_tiles(c);
     const dim3 grid(tile_march_blocks(tm)), block(BOX_X, FROWS);
     const bool ref = !periodic(c, 0) || !periodic(c, 1) || !periodic(c, 2);
-    const auto kern = lam_part ? (ref ? k_visc_fluxes<T, true, true> : k_visc_fluxes<T, true, false>)
-                               : (ref ? k_visc_fluxes<T, false, true> : k_visc_fluxes<T, false, false>);
-    kern<<<grid, block, 0, b->stream>>>(c, tm, b->prim, b->met, vf, lam_part);
+    if (q && (ref || lam_part)) return fail(b, CBNS_ERR_STATE, "flux pass from Q: periodic, no dt");
+    const auto kern =
+        q ? k_visc_fluxes<T, false, false, true>
+          : (lam_part ? (ref ? k_visc_fluxes<T, true, true, false> : k_visc_fluxes<T, true, false, false>)
+                      : (ref ? k_visc_fluxes<T, false, true, false>
+                             : k_visc_fluxes<T, false, false, false>));
+    kern<<<grid, block, 0, b->stream>>>(c, tm, b->prim, q, b->met, vf, lam_part);
     CBNS_HIP(b, hipGetLastError());
   }
   if (!(parts & 2)) return CBNS_OK;
@@ -424,13 +462,15 @@ int viscous(cbns_block* b, T* vf, double* out, int mode, double* lam_part, int p
   return CBNS_OK;
 }
 
-int launch_viscous(cbns_block* b, double* vf, double* out, int mode, double* lam_part, int parts) {
-  return viscous<double>(b, vf, out, mode, lam_part, parts);
+int launch_viscous(cbns_block* b, double* vf, double* out, int mode, double* lam_part, int parts,
+                   const double* q) {
+  return viscous<double>(b, vf, out, mode, lam_part, parts, q);
 }
 
 // precision form: the same scratch holds 12*S floats
-int launch_viscous_f32(cbns_block* b, double* scratch, double* rhs, double* lam_part, int parts) {
-  return viscous<float>(b, reinterpret_cast<float*>(scratch), rhs, 1, lam_part, parts);
+int launch_viscous_f32(cbns_block* b, double* scratch, double* rhs, double* lam_part, int parts,
+                       const double* q) {
+  return viscous<float>(b, reinterpret_cast<float*>(scratch), rhs, 1, lam_part, parts, q);
 }
 
 }  // namespace cbns
