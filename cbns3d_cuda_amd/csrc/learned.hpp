@@ -54,6 +54,18 @@ __device__ __forceinline__ short f32_to_bf16(float x) {
   return __builtin_bit_cast(short, (__bf16)x);
 }
 
+// two at once, a in the low half: one instruction, where two conversions and a
+// merge took four
+__device__ __forceinline__ int pack_bf16(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(int, __builtin_convertvector((f32x2){a, b}, bf2));
+}
+__device__ __forceinline__ bf16x4 pack_bf16x4(float a, float b, float c, float d) {
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(bf16x4, (i32x2){pack_bf16(a, b), pack_bf16(c, d)});
+}
+
 // max(x, 0) on the bit pattern: negative floats (and -0) are negative
 // integers, so one integer max is the ReLU
 __device__ __forceinline__ float relu(float x) {
@@ -181,7 +193,7 @@ __device__ __forceinline__ float mlp_logit_wave(const float x[MLP_IN], const Mlp
     int* row = reinterpret_cast<int*>(lds + l * MLP_IN);
 #pragma unroll
     for (int c = 0; c < MLP_IN / 2; c++)
-      row[c] = (int)(uint16_t)f32_to_bf16(x[2 * c]) | ((int)f32_to_bf16(x[2 * c + 1]) << 16);
+      row[c] = pack_bf16(x[2 * c], x[2 * c + 1]);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -213,12 +225,8 @@ __device__ __forceinline__ float mlp_logit_wave(const float x[MLP_IN], const Mlp
     z0 = mfma_bf16(a11, x1, z0);
     f32x4 z1 = mfma_bf16(a12, x0, c11);
     z1 = mfma_bf16(a13, x1, z1);
-    bf16x4 h0, h1;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      h0[v] = f32_to_bf16(relu(z0[v]));
-      h1[v] = f32_to_bf16(relu(z1[v]));
-    }
+    const bf16x4 h0 = pack_bf16x4(relu(z0[0]), relu(z0[1]), relu(z0[2]), relu(z0[3]));
+    const bf16x4 h1 = pack_bf16x4(relu(z1[0]), relu(z1[1]), relu(z1[2]), relu(z1[3]));
     f32x4 y0 = mfma_bf16(a20, h0, c20);
     y0 = mfma_bf16(a21, h1, y0);
     f32x4 y1 = mfma_bf16(a22, h0, c21);
