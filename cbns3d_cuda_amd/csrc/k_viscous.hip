@@ -60,7 +60,11 @@ constexpr int VROWS = VISC_ROWS;
 // latency a plane (2 us on an idle chip, 4 planes of lead-in on top), so the
 // best length is short: 5 of 1, 2, 3, 4, 5, 6, 8, 12, 16, 32 at 64^3 to 256^3
 // (128^3 FP64 134 us, 137 at 4, 143 at 12; 256^3 1023, 1040 at 8, 1064 at 12),
-// 2 where 5 would leave fewer than 448 workgroups (32^3: 11 us, 16 at 5).
+// 2 where 5 would leave fewer than 448 workgroups (32^3: 11 us, 16 at 5; 64^3, 476
+// of them, 26.5, 28.7 at 2), or, with reference axes, whose kernel runs two a CU,
+// just over 512: a second round nearly empty (us at 5 / 2: FP32 456 of them 28.5 /
+// 30.9, 520 34.6 / 29.8, FP64 520 38 / 34, 193x61x33 with 544 37 / 34, 130x100x30 with
+// 546 39 / 39).
 constexpr int VISC_FLUX_CHUNK = 5, VISC_FLUX_CHUNK_SMALL = 2;
 constexpr int FROWS = VISC_FLUX_ROWS;
 
@@ -420,7 +424,9 @@ static TileMarch visc_flux_tiles(const Consts& c) {
     vb.n[a] = axis_n(c, a) + 4;
   }
   const TileMarch tm = tile_march(vb, VISC_FLUX_CHUNK, FROWS, 2);
-  if ((long)tm.ntx * tm.nty * tm.nkc >= 448) return tm;
+  const bool ref = !periodic(c, 0) || !periodic(c, 1) || !periodic(c, 2);
+  const long nb = (long)tm.ntx * tm.nty * tm.nkc;
+  if (nb >= 448 && !(ref && nb > 512 && nb < 576)) return tm;
   return tile_march(vb, VISC_FLUX_CHUNK_SMALL, FROWS, 2);
 }
 
