@@ -85,7 +85,9 @@ def kernel_work(name, p):
         return "byte", sum(faces) // 3 * (5 + 8) * 8
     # ghost shell of 4 layers: Q (5) + the primitives the stage wrote, read
     # and written; averaged over a step (stages 1-2: u, v, w, T on viscous
-    # blocks, none on inviscid ones; stage 3: all)
+    # blocks with boundary rules, none on inviscid ones; stage 3: all).  Periodic
+    # viscous steps, counted alike, refresh no primitives in stages 1-2 either:
+    # their rate here is stated 29/21 of what it is.
     fields = (2 * 9 + 11) / 3 if p.viscous else (2 * 5 + 10) / 3
     shell = (p.IM + 8) * (p.JM + 8) * (p.KM + 8) - p.IM * p.JM * p.KM
     return "byte", int(shell * fields * 16)
@@ -135,8 +137,8 @@ def step_hbm(kt, steps, ms_step, p, workload):
     gbs = total / (ms_step / 1e3) / 1e9
     return {"bytes_per_step": total, "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": gbs / PEAK_HBM_GBS,
-            "note": "measured HBM bytes per step (the viscous flux pass at its bytes without "
-                    "the time-step maxima, 6 % fewer than the first stage's) over ms_per_step"}
+            "note": "measured HBM bytes per step (each kernel's averaged over a step's "
+                    "launches) over ms_per_step"}
 
 
 def log(*a):
