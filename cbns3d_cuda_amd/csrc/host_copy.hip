@@ -106,6 +106,18 @@ struct Copy {
   }
 };
 
+// Memory that HIP does not know, as malloc returns it.  What a caller has pinned
+// (or allocated on a device) is the runtime's to copy to: it writes pinned memory
+// over the link at once, and the ring would add a pass of the host over every byte
+// (one field into pinned memory, ring / runtime: 0.65 / 0.37 ms at 20 MB, 1.9 / 1.4
+// at 76 MB).
+bool ordinary_memory(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
+
 // the ring's way; false if it could not be taken (nothing copied, or not all)
 bool ring_copy(hipStream_t s, const void* dev, void* host, size_t bytes) {
   std::unique_lock<std::mutex> lock(ring.mu, std::try_to_lock);
@@ -158,7 +170,8 @@ void host_copy_unref() {
 }
 
 int copy_to_host(cbns_block* b, const void* dev, void* host, size_t bytes) {
-  if (bytes >= LEAST && ring_copy(b->stream, dev, host, bytes)) return CBNS_OK;
+  if (bytes >= LEAST && ordinary_memory(host) && ring_copy(b->stream, dev, host, bytes))
+    return CBNS_OK;
   CBNS_HIP(b, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, b->stream));
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   return CBNS_OK;
