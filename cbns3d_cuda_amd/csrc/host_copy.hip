@@ -170,8 +170,12 @@ void host_copy_unref() {
 }
 
 int copy_to_host(cbns_block* b, const void* dev, void* host, size_t bytes) {
-  if (bytes >= LEAST && ordinary_memory(host) && ring_copy(b->stream, dev, host, bytes))
-    return CBNS_OK;
+  if (bytes >= LEAST && ordinary_memory(host)) {
+    // what is queued ahead of the copy is waited for by this thread alone: the ring's
+    // would poll all that time, and other blocks' copies would find the ring taken
+    CBNS_HIP(b, hipStreamSynchronize(b->stream));
+    if (ring_copy(b->stream, dev, host, bytes)) return CBNS_OK;
+  }
   CBNS_HIP(b, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, b->stream));
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   return CBNS_OK;

@@ -1,9 +1,9 @@
 """What a read-back of fields costs the host (csrc/host_copy.hip).  The ring and its
 threads are for ordinary memory: a copy into memory that HIP knows (pinned by the
-caller) goes there directly.  It shows in the processor time of the read over its
-own duration: one waiting thread uses at most the duration, and the runtime's own
-thread as much again; eight threads use up to eight times it.  The bound of 3 lies
-between.
+caller) goes there directly, and while the stream still has work none of the threads
+runs.  Both show in the processor time of the read over its own duration: one waiting
+thread uses at most the duration, and the runtime's own thread as much again; eight
+threads use up to eight times it.  The bound of 3 lies between.
 """
 import ctypes as C
 import resource
@@ -67,4 +67,22 @@ def test_pinned_destination_takes_no_threads():
     finally:
         if p:
             hip.hipHostFree(p)
+        b.free()
+
+
+def test_queued_work_is_waited_for_by_one_thread():
+    b = _block(64)
+    try:
+        b.get_field(F_Q, 5)  # the ring is there
+        for _ in range(400):
+            for s in (1, 2, 3):
+                b.rk3_stage(0.0, s)
+        out = []
+        t0 = time.perf_counter()
+        busy = _threads_busy(lambda: out.append(b.get_field(F_Q, 5)))
+        print("read took", time.perf_counter() - t0, "threads busy", busy, flush=True)
+        assert time.perf_counter() - t0 > 0.01  # the stages were still queued
+        assert np.isfinite(out[0]).all()
+        assert busy < 3.0
+    finally:
         b.free()
