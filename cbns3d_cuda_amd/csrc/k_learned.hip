@@ -18,6 +18,7 @@
 //   k_mlp_pack          fp32 parameters -> bf16 operand tiles
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "cbns_internal.hpp"
@@ -497,7 +498,11 @@ struct cbns_mlp {
   float* v = nullptr;
   cbns::bf16x4* pack = nullptr;  // 3 x 256 operand tiles
   float* part = nullptr;         // GRAD_BLOCKS rows of a gradient pass
-  float* host = nullptr;         // pinned: a gradient and its loss, or the parameters
+  // pinned: a gradient and its loss, or the parameters; a call holds host_mu from its
+  // launches until it has read what they left there, so that two threads' calls on
+  // one network do not read each other's
+  float* host = nullptr;
+  std::mutex host_mu;
   int t = 0;                     // Adam step count
   std::string err;
 };
@@ -590,6 +595,7 @@ int cbns_mlp_set_params(cbns_mlp* m, const float* params) {
 int cbns_mlp_get_params(cbns_mlp* m, float* params) {
   if (!m || !params) return CBNS_ERR_ARG;
   const size_t nb = cbns::MLP_NPARAM * sizeof(float);
+  std::lock_guard<std::mutex> lock(m->host_mu);
   MLP_HIP(m, hipMemcpyAsync(m->host, m->P, nb, hipMemcpyDeviceToHost, m->stream));
   MLP_HIP(m, hipStreamSynchronize(m->stream));
   std::memcpy(params, m->host, nb);
@@ -615,6 +621,7 @@ int cbns_mlp_loss_grad(cbns_mlp* m, const float* feat, const float* target, int6
                                          cbns::GRAD_BLOCKS);
   const long per_it = (long)blocks * cbns::GRAD_WAVES;
   const int iters = (int)((tiles + per_it - 1) / per_it);
+  std::lock_guard<std::mutex> lock(m->host_mu);
   cbns::k_mlp_grad<<<blocks, 64 * cbns::GRAD_WAVES, 0, m->stream>>>(
       mlp_dev(m), feat, target, n, w_pos, 1.0f / (float)n, iters, m->part);
   MLP_HIP(m, hipGetLastError());
