@@ -64,6 +64,7 @@ struct Copy {
   char* host;
   size_t bytes, piece;
   int buffers, pieces;
+  int issued = 0;              // pieces on their way into the ring, or past it
   std::atomic<int> next{0};    // piece the next free worker takes
   std::atomic<int> landed{0};  // pieces that have arrived in the ring
   std::atomic<bool> failed{false};
@@ -82,23 +83,27 @@ struct Copy {
       out[p].store(true, std::memory_order_release);
     }
   }
+  // issues the pieces that piece p's turn leaves room for; false after a HIP error
+  bool issue(int p, hipStream_t s, Events& e) {
+    for (; issued < pieces && issued < p + buffers; issued++) {
+      if (issued >= buffers) {
+        // has the buffer's last piece left it?  Only the piece that is due
+        // next is waited for: the others can be issued a round later
+        if (issued > p && !out[issued - buffers].load(std::memory_order_acquire)) break;
+        while (!out[issued - buffers].load(std::memory_order_acquire)) std::this_thread::yield();
+      }
+      const int b = issued % buffers;
+      if (hipMemcpyAsync(ring.buf + b * piece, dev + issued * piece, size(issued),
+                         hipMemcpyDeviceToHost, s) != hipSuccess ||
+          hipEventRecord(e.ev[b], s) != hipSuccess)
+        return false;
+    }
+    return true;
+  }
   // moves the pieces into the ring; false after a HIP error
   bool feed(hipStream_t s, Events& e) {
-    int issued = 0;
     for (int p = 0; p < pieces; p++) {
-      for (; issued < pieces && issued < p + buffers; issued++) {
-        if (issued >= buffers) {
-          // has the buffer's last piece left it?  Only the piece that is due
-          // next is waited for: the others can be issued a round later
-          if (issued > p && !out[issued - buffers].load(std::memory_order_acquire)) break;
-          while (!out[issued - buffers].load(std::memory_order_acquire)) std::this_thread::yield();
-        }
-        const int b = issued % buffers;
-        if (hipMemcpyAsync(ring.buf + b * piece, dev + issued * piece, size(issued),
-                           hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipEventRecord(e.ev[b], s) != hipSuccess)
-          return false;
-      }
+      if (!issue(p, s, e)) return false;
       if (hipEventSynchronize(e.ev[p % buffers]) != hipSuccess) return false;
       landed.store(p + 1, std::memory_order_release);
     }
@@ -125,6 +130,7 @@ bool ring_copy(hipStream_t s, const void* dev, void* host, size_t bytes) {
   Events e;
   Copy c;
   std::vector<std::thread> threads;
+  bool ok = false;
   try {
     if (!ring.buf && hipHostMalloc((void**)&ring.buf, RING, hipHostMallocPortable) != hipSuccess) {
       ring.buf = nullptr;
@@ -143,11 +149,13 @@ bool ring_copy(hipStream_t s, const void* dev, void* host, size_t bytes) {
     const unsigned cores = std::max(2u, std::thread::hardware_concurrency());
     const int n = std::min({MAX_THREADS, c.pieces, (int)(cores / 2)});
     threads.reserve(n);
-    for (int t = 0; t < n; t++) threads.emplace_back([&c] { c.work(); });
-  } catch (...) {  // no memory or no thread: those that run are let go
-    if (threads.empty()) return false;
+    // the first pieces are on their way while the threads start
+    ok = c.issue(0, s, e);
+    for (int t = 0; ok && t < n; t++) threads.emplace_back([&c] { c.work(); });
+  } catch (...) {  // no memory or no thread: those that run do the copy
+    if (threads.empty()) ok = false;
   }
-  const bool ok = c.feed(s, e);
+  ok = ok && c.feed(s, e);
   if (!ok) c.failed.store(true);
   for (std::thread& t : threads) t.join();
   if (!ok) (void)hipStreamSynchronize(s);  // nothing writes the ring any more
