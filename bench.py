@@ -36,13 +36,14 @@ PEAK_HBM_GBS = 8000.0
 # with an operation-counting scalar (make -C oracle opcount && oracle/opcount).
 FLOPS_PER_FACE = 1580.0
 # Algorithmic HBM bytes of the memory-bound kernels (compulsory traffic, each
-# value moved once): viscous fluxes read u,v,w,T and the 10 metrics and write
-# Ev,Fv,Gv (12) per node of the viscous range (N+4)^3; a divergence pass
+# value moved once): viscous fluxes read u,v,w,T (or the five of Q) and the 10
+# metrics and write Ev,Fv,Gv (12) per node of the viscous range (N+4)^3, and a
+# step's first pass reads rho and p too, for dt; a divergence pass
 # (reference-decomposed calls only: the fused stage's marches take the
 # divergence) reads the 12 fluxes and read-modify-writes the 4
 # momentum/energy rhs components per updated node; dt reads 6 primitives and
 # 9 metrics per node.
-VISC_FLUX_BYTES_PER_NODE = (4 + 10 + 12) * 8
+VISC_FLUX_BYTES_PER_NODE = (10 + 12) * 8  # its 4 to 6 state fields come on top
 VISC_DIV_BYTES_PER_NODE = (12 + 2 * 4) * 8
 DT_BYTES_PER_NODE = (6 + 9) * 8
 
@@ -62,8 +63,29 @@ def face_counts(p):
     return faces, upd
 
 
-def kernel_work(name, p):
-    """(kind, units of work per launch) for the per-kernel roofline."""
+def as_run(p, kt):
+    """How the library runs the steps of block p (kernel_work's keywords): kt, the
+    profiled pass, tells tiles (whose launch is booked under march_zeta, and none
+    under march_eta) from marches; the flux pass's choices follow the rules of
+    flux_pass_from_q (csrc/cbns_internal.hpp) and visc_flux_tiles (csrc/k_viscous.hip)."""
+    periodic = all(p.bc[a] == 1 for a in range(3))
+    n = flux_pass_groups(p, 5)
+    short = n < 448 or (not periodic and 512 < n < 576)
+    return {"tiles": kt["march_zeta"][1] > 0 and kt["march_eta"][1] == 0,
+            "from_q": bool(p.viscous) and periodic, "planes": 2 if short else 5}
+
+
+def flux_pass_groups(p, planes):
+    """Workgroups of the viscous flux pass: 60 x 4 nodes by `planes` along k."""
+    return ((p.IM + 4 + 59) // 60) * ((p.JM + 4 + 3) // 4) * -(-(p.KM + 4) // planes)
+
+
+def kernel_work(name, p, tiles=False, from_q=False, planes=8):
+    """(kind, units of work per launch) for the per-kernel roofline, averaged over
+    a step's launches.  tiles: a stage is one launch over tiles, all three axes'
+    faces in it.  from_q: the flux passes of stages 2 and 3 read the five fields of
+    the stage input, and stages 1 and 2 leave no primitives.  planes: nodes along k
+    of a flux-pass workgroup."""
     faces, upd = face_counts(p)
     nodes = upd[0] * upd[1] * upd[2]
     if name == "march_eta":  # eta-faces
@@ -71,24 +93,24 @@ def kernel_work(name, p):
     if name == "xfaces":
         return "flop", faces[0] * FLOPS_PER_FACE
     if name == "march_zeta":  # xi- and zeta-faces (xi fused into the zeta march)
-        return "flop", (faces[0] + faces[2]) * FLOPS_PER_FACE
+        return "flop", (faces[0] + faces[2] + (faces[1] if tiles else 0)) * FLOPS_PER_FACE
     if name == "visc_flux":
-        return "byte", (p.IM + 4) * (p.JM + 4) * (p.KM + 4) * VISC_FLUX_BYTES_PER_NODE
+        ext = (p.IM + 4) * (p.JM + 4) * (p.KM + 4)
+        fields = (4 + 5 + 5) if from_q else (4 + 4 + 4)
+        return "byte", (ext * (3 * VISC_FLUX_BYTES_PER_NODE + fields * 8) +
+                        p.IM * p.JM * p.KM * 2 * 8) // 3
     if name == "visc_div":
         return "byte", nodes * VISC_DIV_BYTES_PER_NODE
     if name == "dt":
         if p.viscous:  # the final pass over the viscous flux pass's maxima
-            n = [(p.IM + 4 + 59) // 60, (p.JM + 4 + 3) // 4, (p.KM + 4 + 7) // 8]
-            return "byte", n[0] * n[1] * n[2] * 8
+            return "byte", flux_pass_groups(p, planes) * 8
         return "byte", p.IM * p.JM * p.KM * DT_BYTES_PER_NODE
     if name == "indicator":  # per axis launch: 6-node stencil + 2 node states read once, 1 B out
         return "byte", sum(faces) // 3 * (5 + 8) * 8
     # ghost shell of 4 layers: Q (5) + the primitives the stage wrote, read
     # and written; averaged over a step (stages 1-2: u, v, w, T on viscous
-    # blocks with boundary rules, none on inviscid ones; stage 3: all).  Periodic
-    # viscous steps, counted alike, refresh no primitives in stages 1-2 either:
-    # their rate here is stated 29/21 of what it is.
-    fields = (2 * 9 + 11) / 3 if p.viscous else (2 * 5 + 10) / 3
+    # blocks with boundary rules, none on others; stage 3: all).
+    fields = (2 * (5 if from_q else 9) + 11) / 3 if p.viscous else (2 * 5 + 10) / 3
     shell = (p.IM + 8) * (p.JM + 8) * (p.KM + 8) - p.IM * p.JM * p.KM
     return "byte", int(shell * fields * 16)
 
@@ -106,8 +128,8 @@ def measured_traffic(name, p, workload):
     return t.get(name)
 
 
-def roofline_of(name, ms, n, p, workload):
-    kind, work = kernel_work(name, p)
+def roofline_of(name, ms, n, p, workload, run):
+    kind, work = kernel_work(name, p, **run)
     avg_s = ms / n / 1e3
     if kind == "flop":
         ach = work / avg_s / 1e12
@@ -115,7 +137,8 @@ def roofline_of(name, ms, n, p, workload):
                 "frac": ach / PEAK_FP64_TFLOPS, "traffic": measured_traffic(name, p, workload),
                 "kernel": name, "avg_ms": ms / n,
                 "note": "FP64 vector-ALU-bound face-flux sweep (no matrix-core work); "
-                        "peak = MI355X FP64 vector"}
+                        "peak = MI355X FP64 vector; achieved counts the operations of the "
+                        "reference's method, of which the kernel executes fewer"}
     ach = work / avg_s / 1e9
     return {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": ach / PEAK_HBM_GBS, "traffic": measured_traffic(name, p, workload),
@@ -360,8 +383,9 @@ def main():
     # dominant kernel and its algorithmic work per launch; every kernel's
     # roofline is listed beside it
     dom = max(kt, key=lambda k: kt[k][0])
-    roof = roofline_of(dom, kt[dom][0], kt[dom][1], p, wl)
-    per_kernel = {k: roofline_of(k, ms, n, p, wl) for k, (ms, n) in kt.items() if n}
+    run = as_run(p, kt)
+    roof = roofline_of(dom, kt[dom][0], kt[dom][1], p, wl, run)
+    per_kernel = {k: roofline_of(k, ms, n, p, wl, run) for k, (ms, n) in kt.items() if n}
     hbm = step_hbm(kt, args.profile_steps, ms_step, p, wl)
 
     forms = None
