@@ -4,9 +4,9 @@
 // host thread, which also takes the page faults of a fresh destination: 10 to
 // 14 GB/s on the machine this is written for, where the link moves 50.  Here
 // the pieces of a large copy go through a ring of pinned buffers that several
-// threads empty.  Five fields into fresh memory, before and after: 0.32 -> 0.27
-// ms at 4.4 MB (40^3), 1.04 -> 0.73 at 15 MB (64^3), 9.9 -> 3.0 at 101 MB
-// (128^3), 70 -> 17 at 736 MB (256^3).  What bounds the large copy is the link
+// threads empty.  Five fields into fresh memory, before and after: 0.27 -> 0.25
+// ms at 4.4 MB (40^3), 1.0 -> 0.70 at 15 MB (64^3), 9.6 -> 3.3 at 101 MB
+// (128^3), 68 -> 20 at 736 MB (256^3).  What bounds the large copy is the link
 // and about 14 us between two pieces; the small one, the start of the threads.
 // The ring is shared by the blocks of the process (16 MiB, given back with the
 // last of them) and used by one copy at a time; a copy that finds it taken, or
@@ -28,9 +28,15 @@ namespace {
 
 constexpr size_t RING = 16u << 20;
 constexpr int MAX_THREADS = 8;  // 4 and 12 are within the noise of 8
-// Copies below this go the runtime's way: at 2.6 MB (32^3) its 0.18 ms are no
+// Copies below this go the runtime's way: at 2.6 MB (32^3) its 0.15 ms are no
 // more than the ring's.
 constexpr size_t LEAST = 4u << 20;
+// Such a copy goes in parts below 1 MiB, from where on the runtime pins the
+// destination for the copy instead of staging it: five fields into memory fresh from
+// the kernel, one by one / one copy / parts, us: 24^3 292 / 316 / 262, 32^3 528 / 618 /
+// 498, 38^3 766 / 924 / 740; into memory used before 105 / 80 / 72, 155 / 148 / 128, 207 /
+// 219 / 186.
+constexpr size_t PART = 1020u << 10;
 // Bytes of a piece.  2 MiB fill the pipeline sooner (0.27 ms against 0.35 at
 // 4.4 MB), 4 MiB have fewer gaps (43 GB/s against 38 at 736 MB; 1 MiB 30).
 inline size_t piece_of(size_t bytes) { return bytes < (32u << 20) ? 2u << 20 : 4u << 20; }
@@ -178,13 +184,22 @@ void host_copy_unref() {
 }
 
 int copy_to_host(cbns_block* b, const void* dev, void* host, size_t bytes) {
-  if (bytes >= LEAST && ordinary_memory(host)) {
+  const bool ordinary = bytes > PART && ordinary_memory(host);
+  size_t parts = 1;
+  if (ordinary && bytes >= LEAST) {
     // what is queued ahead of the copy is waited for by this thread alone: the ring's
     // would poll all that time, and other blocks' copies would find the ring taken
     CBNS_HIP(b, hipStreamSynchronize(b->stream));
     if (ring_copy(b->stream, dev, host, bytes)) return CBNS_OK;
+  } else if (ordinary) {
+    parts = (bytes + PART - 1) / PART;
   }
-  CBNS_HIP(b, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, b->stream));
+  for (size_t p = 0; p < parts; p++) {
+    const size_t from = bytes * p / parts, to = bytes * (p + 1) / parts;
+    CBNS_HIP(b, hipMemcpyAsync(static_cast<char*>(host) + from,
+                               static_cast<const char*>(dev) + from, to - from,
+                               hipMemcpyDeviceToHost, b->stream));
+  }
   CBNS_HIP(b, hipStreamSynchronize(b->stream));
   return CBNS_OK;
 }
