@@ -26,9 +26,15 @@
 //     sqrt costs ~11-12 VALU instructions on gfx950, this 3-4, and a second
 //     step (<= 1.4e-16) would cost 2-3 more in a VALU-bound sweep.
 //     Arguments are positive and finite wherever they are used.
-// Every sum of products names its fused operations, so a face has the same bits
-// in whichever kernel forms it; in the precision form a last bit of a float, or a
-// double next to one, shows in the step's result.
+// Every sum of products names its fused operations, so a face's bits do not depend
+// on the code around it, and the marches and the tiles form it alike.  Some functions
+// take which product of a sum is rounded (yz, CHAIN, SWAP; k_fused.hip's Rounding):
+// in the precision and hybrid forms a last bit of a float, or a double next to one,
+// shows in the step's result, and these keep the results that those forms have had.
+// So the WENO lists of a hybrid round a listed face otherwise than a march would, and
+// in these two forms the face at every 32nd node of an eta or zeta line is rounded
+// otherwise for the node before it than for the node after it: their update conserves
+// there to rounding only.
 // The result equals the reference formula up to rounding (the stage parity
 // bar is 1e-12 relative; tests/test_gpu_parity.py).
 #pragma once
@@ -288,8 +294,8 @@ __device__ __forceinline__ void weno5_pair(double e01, double e12, double e23, d
             fma(2.0 / 3.0, da, e12), fma(2.0, e12, four), four - e34, nl, dl);
   weno5_sum(fma(k13 * df, df, fma(r2, r2, eps)), fma(r4, r4, td), fma(r6, r6, tc),
             fma(-2.0 / 3.0, df, e34), fma(2.0, e34, four), four - e12, nr, dr);
-  // one reciprocal for both sides: dl, dr lie in [1e-22, 1e123] for any
-  // smoothness indicator below 1e30, so dl dr stays in range
+  // one reciprocal for both sides: dl, dr lie in [2e-21, 3e123] for any
+  // smoothness indicator (four times as large here) below 1e30, so dl dr stays in range
   const double x = 0.5 * fast_rcp(dl * dr);
   left = nl * (dr * x);
   right = -nr * (dl * x);
@@ -320,7 +326,7 @@ __device__ __forceinline__ void weno5_pair_dev(float w0, float w1, float w3, flo
 // (nx,ny,nz) the unnormalised face vector 0.5 (J grad xi |_m + J grad xi |_{m+1}).
 // Against projecting the six node states and taking each field's differences
 // afterwards the face has 25 differences and a sixth of the projections fewer: the
-// marches' loops go from 724 to 685 FP64 operations a face.
+// eta march's loop goes from 731 FP64 instructions to 696.
 __device__ __forceinline__ void face_flux_basis(const GasT<double>& g, const double e[5][5],
                                                 const double qm[5], const double qp[5],
                                                 const Basis<double>& B, double nx, double ny,

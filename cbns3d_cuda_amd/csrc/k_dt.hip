@@ -68,7 +68,8 @@ __global__ void __launch_bounds__(TPB) k_time_step(Consts c, int chunk,
 // The host's copy goes to pinned memory from here: a copy of its own behind the
 // kernels took 1.6 us of a 24^3 step (43.1 -> 41.5), 4 of a viscous one (67 -> 63).
 // (one workgroup; eight independent loads a thread in flight: 23 -> 9 us for
-// the 10,890 maxima of a 256^3 flux pass, with 256 threads and one load before)
+// the 10,890 maxima that a 256^3 flux pass then left (16,900 now), with 256 threads
+// and one load before)
 __global__ void __launch_bounds__(FINAL_TPB) k_dt_final(const double* __restrict__ partial, int n,
                                                         double CFL, double cap,
                                                         double* __restrict__ out,

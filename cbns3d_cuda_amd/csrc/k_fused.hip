@@ -541,7 +541,8 @@ k_march(Consts c, StageArgs sa, const double* __restrict__ met) {
 // the tile's nodes from them.  The faces between tiles are formed twice, but no
 // lane waits for another's faces and dF stays out of memory, so blocks that are
 // small for the marches run this way (stage_shape).  A face's operations are the
-// marches', so the stage has their bits.
+// marches', so the stage has their bits (for that it also rounds the face at every
+// 32nd node as the march that opens a chunk of CHUNK_MAX there: first_on_line).
 
 // The tile of this workgroup (X x Y x Z nodes from lo on, nx x ny x nz of them in
 // the block); false past the last.  Workgroups go to the 8 XCDs in turn; each XCD

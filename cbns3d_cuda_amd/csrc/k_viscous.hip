@@ -64,7 +64,8 @@ constexpr int VROWS = VISC_ROWS;
 // of them, 26.5, 28.7 at 2), or, with reference axes, whose kernel runs two a CU,
 // just over 512: a second round nearly empty (us at 5 / 2: FP32 456 of them 28.5 /
 // 30.9, 520 34.6 / 29.8, FP64 520 38 / 34, 193x61x33 with 544 37 / 34, 130x100x30 with
-// 546 39 / 39).
+// 546 39 / 39; from there to 576 nothing was measured, and a third round, past 1024,
+// is a smaller part of the pass and left as it is).
 constexpr int VISC_FLUX_CHUNK = 5, VISC_FLUX_CHUNK_SMALL = 2;
 constexpr int FROWS = VISC_FLUX_ROWS;
 

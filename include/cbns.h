@@ -166,12 +166,14 @@ int64_t cbns_field_size(const cbns_block* blk);
  * the summed milliseconds and launch count of one kernel id since the last
  * reset and reset=1 clears it. */
 enum {
-  CBNS_K_XFACES = 0,     /* xi-face fluxes                          */
-  CBNS_K_MARCH_ETA = 1,  /* eta sweep (+ Fv's divergence)           */
-  CBNS_K_MARCH_ZETA = 2, /* zeta + xi sweep (+ Gv's, Ev's divergence) + RK stage combination */
+  CBNS_K_XFACES = 0,     /* xi-face fluxes (no launch of its own: in CBNS_K_MARCH_ZETA) */
+  CBNS_K_MARCH_ETA = 1,  /* eta sweep (+ Fv's divergence); no launch on blocks that run by tiles */
+  CBNS_K_MARCH_ZETA = 2, /* zeta + xi sweep (+ Gv's, Ev's divergence) + RK stage combination;
+                            on blocks that run by tiles the whole stage: the faces of all axes,
+                            the combination and, on small periodic blocks, the ghosts */
   CBNS_K_VISC_FLUX = 3,  /* viscous fluxes Ev,Fv,Gv at the nodes     */
   CBNS_K_VISC_DIV = 4,   /* viscous divergence pass (reference-decomposed calls; the fused stage has none) */
-  CBNS_K_BC = 5,         /* boundary / ghost fill                   */
+  CBNS_K_BC = 5,         /* boundary / ghost fill; no launch where the tiles write the ghosts */
   CBNS_K_DT = 6,         /* CFL time step reduction                 */
   CBNS_K_INDICATOR = 7,  /* learned troubled-face flags (hybrid)    */
   CBNS_K_WENO_LIST = 8,  /* WENO fluxes of the troubled faces (hybrid) */
