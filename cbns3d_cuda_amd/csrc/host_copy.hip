@@ -4,13 +4,13 @@
 // host thread, which also takes the page faults of a fresh destination: 10 to
 // 14 GB/s on the machine this is written for, where the link moves 50.  Here
 // the pieces of a large copy go through a ring of pinned buffers that several
-// threads empty.  Five fields into fresh memory, before and after: 0.27 -> 0.25
-// ms at 4.4 MB (40^3), 1.0 -> 0.70 at 15 MB (64^3), 9.6 -> 3.3 at 101 MB
+// threads empty.  Five fields into fresh memory, before and after: 0.28 -> 0.26
+// ms at 4.4 MB (40^3), 1.0 -> 0.73 at 15 MB (64^3), 9.6 -> 3.3 at 101 MB
 // (128^3), 68 -> 20 at 736 MB (256^3).  What bounds the large copy is the link
 // and about 14 us between two pieces; the small one, the start of the threads.
-// The ring is shared by the blocks of the process (16 MiB, given back with the
-// last of them) and used by one copy at a time; a copy that finds it taken, or
-// no threads to be had, goes the runtime's way.
+// The ring is shared by the blocks of the process (16 MiB, made once they have read
+// enough and given back with the last of them) and used by one copy at a time; a
+// copy that finds it taken, or no threads to be had, goes the runtime's way.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -31,12 +31,20 @@ constexpr int MAX_THREADS = 8;  // 4 and 12 are within the noise of 8
 // Copies below this go the runtime's way: at 2.6 MB (32^3) its 0.15 ms are no
 // more than the ring's.
 constexpr size_t LEAST = 4u << 20;
-// Such a copy goes in parts below 1 MiB, from where on the runtime pins the
+// Bytes read since the last ring was given back that are worth a new one.  Its pinned
+// memory takes 1.5 ms to make where the runtime does not hold some, and given back
+// it takes the place of a block's arrays among what the runtime holds.  A program
+// that makes a block of 64^3, reads its state once (15 MB) and frees it, again and
+// again, waited 2.3 ms for the read with a ring each time, 1.1 without; the ring saves
+// 0.3 of them.  A copy of 64 MiB pays for it at once.
+constexpr size_t WORTH = 64u << 20;
+// A copy without the ring goes in parts below 1 MiB, from where on the runtime pins the
 // destination for the copy instead of staging it: five fields into memory fresh from
 // the kernel, one by one / one copy / parts, us: 24^3 292 / 316 / 262, 32^3 528 / 618 /
 // 498, 38^3 766 / 924 / 740; into memory used before 105 / 80 / 72, 155 / 148 / 128, 207 /
-// 219 / 186.
-constexpr size_t PART = 1020u << 10;
+// 219 / 186.  Up to 32 MiB: 16 MiB fresh / used whole 5.2 / 0.99 ms, in parts 4.4 / 0.90,
+// 48 MiB 15.7 / 2.9 and 14.4 / 3.3.
+constexpr size_t PART = 1020u << 10, MOST_PARTED = 32u << 20;
 // Bytes of a piece.  2 MiB fill the pipeline sooner (0.27 ms against 0.35 at
 // 4.4 MB), 4 MiB have fewer gaps (43 GB/s against 38 at 736 MB; 1 MiB 30).
 inline size_t piece_of(size_t bytes) { return bytes < (32u << 20) ? 2u << 20 : 4u << 20; }
@@ -47,6 +55,7 @@ struct Ring {
   std::mutex refs_mu;
   int refs = 0;
   char* buf = nullptr;
+  size_t without = 0;  // bytes copied since there was no ring, up to WORTH
 };
 Ring ring;
 
@@ -133,6 +142,10 @@ bool ordinary_memory(const void* p) {
 bool ring_copy(hipStream_t s, const void* dev, void* host, size_t bytes) {
   std::unique_lock<std::mutex> lock(ring.mu, std::try_to_lock);
   if (!lock.owns_lock()) return false;
+  if (!ring.buf) {
+    ring.without = std::min(WORTH, ring.without + std::min(bytes, WORTH));
+    if (ring.without < WORTH) return false;
+  }
   Events e;
   Copy c;
   std::vector<std::thread> threads;
@@ -181,19 +194,18 @@ void host_copy_unref() {
   std::lock_guard<std::mutex> use(ring.mu);
   if (ring.buf) (void)hipHostFree(ring.buf);
   ring.buf = nullptr;
+  ring.without = 0;
 }
 
 int copy_to_host(cbns_block* b, const void* dev, void* host, size_t bytes) {
   const bool ordinary = bytes > PART && ordinary_memory(host);
-  size_t parts = 1;
   if (ordinary && bytes >= LEAST) {
     // what is queued ahead of the copy is waited for by this thread alone: the ring's
     // would poll all that time, and other blocks' copies would find the ring taken
     CBNS_HIP(b, hipStreamSynchronize(b->stream));
     if (ring_copy(b->stream, dev, host, bytes)) return CBNS_OK;
-  } else if (ordinary) {
-    parts = (bytes + PART - 1) / PART;
   }
+  const size_t parts = ordinary && bytes <= MOST_PARTED ? (bytes + PART - 1) / PART : 1;
   for (size_t p = 0; p < parts; p++) {
     const size_t from = bytes * p / parts, to = bytes * (p + 1) / parts;
     CBNS_HIP(b, hipMemcpyAsync(static_cast<char*>(host) + from,
